@@ -765,8 +765,10 @@ int prefill_attn_impl(void* out, const void* q, const void* k_cache, const void*
   SKV_REQUIRE(blocks < (1L << 31), SKV_E_UNSUPPORTED, "%s: grid too large", fn);
   if (!launch) return SKV_OK;
   hipStream_t s = (hipStream_t)stream;
-  // LV: 0 = LDS DMA at the exact head dim; 8 = 16-byte register loads; 1 = element loads
-  const int LV = DK == D ? 0 : (D % 8 == 0 ? 8 : 1);
+  // LV: 0 = LDS DMA at an exact head dim of 64, 128 or 256 (a 32-wide row is a quarter
+  // of a DMA piece's lanes and has no such kernel); 8 = 16-byte register loads; 1 = element
+  // loads
+  const int LV = DK == D && D != 32 ? 0 : (D % 8 == 0 ? 8 : 1);
 #define SKV_PF(DD, GG, LL)                                                                    \
   if (DK == DD && G == GG && LV == LL)                                                        \
     hipLaunchKernelGGL((k_prefill_mfma<DD, GG, LL>), dim3((unsigned)blocks),                  \

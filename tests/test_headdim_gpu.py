@@ -246,6 +246,22 @@ def test_prefill_bf16_any_head_dim(gpu_ctx, D, G, n_splits):
     assert not got[~valid].any()
 
 
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("n_splits", [1, 3])
+def test_prefill_bf16_head_dim_32(gpu_ctx, G, n_splits):
+    """A head dim equal to the smallest padded size takes the register-staged
+    kernel and its merge pass (it once matched no attention kernel at all, and
+    the 256-wide merge)."""
+    banner(f"prefill bf16 D=32 G={G} n_splits={n_splits}")
+    got, want, valid, *_ = run_prefill(gpu_ctx, 2, 900, 4 * G, 4, 32, [300, 0], 200,
+                                       n_new=[200, 77], seed=32, n_splits=n_splits)
+    B_, C_, Hq_, D_ = got.shape
+    err = rel_err_rows(got.reshape(B_, C_, Hq_ * D_), want.reshape(B_, C_, Hq_ * D_), valid[..., 0])
+    print(f"rel_err={err:.3e}")
+    assert err < BF16_TOL
+    assert not got[~valid].any()
+
+
 @pytest.mark.parametrize("D", [4, 20, 24, 30, 36, 48, 80, 100, 127, 130, 160, 192, 200, 255, 256])
 def test_prefill_fp32_any_head_dim(gpu_ctx, D):
     banner(f"prefill fp32 D={D}")
