@@ -295,10 +295,12 @@ int skv_layernorm(float* y, const float* x, const float* gamma, const float* bet
  * workgroup of each tile to finish sums the split (arrival counters kept in
  * ws): ws must be zero-filled before its first use, and every call leaves
  * the counters at zero again; with LayerNorm a second kernel sums it.
- * M > 64 (a prompt's prefill): a tiled MFMA GEMM (128 x 128 tiles of
- * v_mfma_f32_32x32x2_f32); with LayerNorm, ws of
- * skv_linear_workspace_bytes(M, N, K) bytes holds the row statistics,
- * computed once (without it every column tile computes its rows' own).
+ * M > 64 (a prompt's prefill): a tiled MFMA GEMM, each fp32 operand as
+ * three bf16 parts and a product as the six partial products of order 2^-16
+ * and larger (fp32 accuracy; operands with infinities take fp32 products);
+ * with LayerNorm, ws (16-byte aligned) of skv_linear_workspace_bytes(M, N,
+ * K) bytes holds the normalised rows, computed once (without it every column
+ * tile normalises its own).
  * Calls that share ws must be stream ordered. */
 int skv_linear(float* y, const float* x, const float* w_t, const float* bias,
                const float* residual, const float* ln_gamma, const float* ln_beta, float ln_eps,
@@ -354,8 +356,8 @@ int skv_linear_packed(float* y, const float* x, const float* w_packed, const flo
 
 /* Workspace skv_linear can use for these sizes: the split-K partials (and
  * arrival counters) of a narrow projection of at most 64 rows (0: it never
- * splits them), or, for more than 64 rows, M * 2 floats of LayerNorm row
- * statistics. Zero-fill it once before the first call. */
+ * splits them), or, for more than 64 rows, M * K floats of normalised
+ * rows. Zero-fill it once before the first call. */
 size_t skv_linear_workspace_bytes(int M, int N, int K);
 
 /* y[m, :] = x[rows[m], :] for m < M, x [n_rows, d] (rows clamped into

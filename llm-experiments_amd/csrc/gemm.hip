@@ -1,22 +1,46 @@
-// Projections over many rows (the model's prompt prefill): a tiled fp32
-// GEMM on MFMA, y = act(LN(x) . w_t^T + bias) + residual, with the
-// semantics of skv_linear (the reference's jnp.dot projections,
-// simple-llm/src/jax_backend.py:110-129, 147, over every position of a
-// window). skv_linear runs this kernel when a call has more than 64 rows;
-// the decode step's few rows stay on k_linear (model_ops.hip), which is
-// bound by reading the weights rather than by the products.
+// Projections over many rows (the model's prompt prefill): a tiled GEMM with
+// fp32 operands and fp32 accuracy on the bf16 matrix cores,
+// y = act(LN(x) . w_t^T + bias) + residual, with the semantics of skv_linear
+// (the reference's jnp.dot projections, simple-llm/src/jax_backend.py:110-129,
+// 147, over every position of a window). skv_linear runs this kernel when a
+// call has more than 64 rows; the decode step's few rows stay on k_linear
+// (model_ops.hip), which is bound by reading the weights rather than by the
+// products.
 //
-// Design: workgroup tile 128 rows x 128 output columns, 4 wavefronts of
-// 64 x 64 (2 x 2 tiles of v_mfma_f32_32x32x2_f32), K in steps of 32. The x
-// and w_t tiles of a step are K-contiguous rows in both operands; they go
-// global -> registers -> LDS ([128][32 + 4] floats each: 16-byte reads of
-// 16 consecutive rows hit distinct banks), and the next step's global
-// loads are issued before the current step's products. A lane reads four
-// consecutive k of its row with one 16-byte LDS load and feeds them to four
-// MFMAs (k = 4*hf + t of each 8-k group, the same permutation for both
-// operands). LayerNorm, when asked for, is applied to the x tile as it is
-// staged, from per-row statistics computed by k_rowstats first (or, without
-// a workspace to hold them, by each workgroup for its own 128 rows).
+// Products: every fp32 operand is split into three bf16 parts, x = h + m + l
+// (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), 8 significant bits
+// each and the differences exact), and a product takes the six partial
+// products of order 2^-16 and larger, hh + hm + mh + mm + hl + lh, on
+// v_mfma_f32_32x32x16_bf16 with fp32 accumulation; what is left out is below
+// 2^-25 of a product. Six bf16 MFMAs do the work of eight
+// v_mfma_f32_32x32x2_f32 in 192 matrix-core cycles instead of 512, and round
+// the accumulator 6 times per 16 k instead of 8.
+// Measured on MI355X against the fp32 MFMA form of the same kernel (128 x 128
+// tiles, one LDS stage): 2048 x 50304 x 768 1390 -> 853 us (186 TFLOP/s),
+// 2048 x 3072 x 768 with LayerNorm 137 -> 67 us, 2048 x 768 x 3072 220 -> 79
+// us, 111 x 640 x 2560 192 -> 48 us; error against float64 (relative
+// 2-norm) 5.0e-7 -> 4.2e-7 at K = 768 and 9.9e-7 -> 8.6e-7 at K = 3072.
+// The split is exact for finite values; an infinity (or a value that rounds
+// to one in bf16) gives a NaN in its rows or columns, so a wavefront whose
+// sums are not all finite computes them again on v_mfma_f32_32x32x2_f32, which
+// gives what fp32 products give.
+//
+// Design: a workgroup computes BM x BN outputs, its wavefronts 64 x 64 or 32
+// x 32 each. K goes in steps of 32: quads of 4 consecutive k are read as fp32
+// two steps ahead, split in registers and stored as three 8-byte pieces, one
+// per plane, into the LDS stage the next step's products read (two stages, one
+// barrier a step). The splitting, 5.5 vector instructions a value, is placed
+// between the MFMAs, which run meanwhile. LDS planes are [rows][32] bf16 with
+// the 16-byte chunks of a row at chunk ^ (row / 4 % 4): 16 rows of one chunk,
+// the operand read, hit 16 distinct 16-byte bank groups. LayerNorm rows are
+// normalised once into the workspace (k_layernorm_rows), or, without one, as
+// they are split. Workgroups that share a weight tile are neighbours on one
+// XCD, so its L2 serves all but the first of them. What bounds it: full tiles
+// run the matrix cores at about 1.1 PFLOP/s of bf16 products (library bf16
+// products reach 1.38 on this card); small calls, the chain of steps of one
+// tile (0.5 us a step for 64 x 64).
+#include <type_traits>
+
 #include "skv_common.h"
 
 namespace skv {
@@ -24,11 +48,13 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kBM = 128, kBN = 128, kBK = 32;
-constexpr int kSP = kBK + 4;  // LDS row stride (floats)
-constexpr int kThreads = 256;
-constexpr int kLoads = kBM * kBK / 4 / kThreads;  // float4 per thread per operand (4)
+constexpr int kBK = 32;  // k per step
+constexpr int kXCD = 8;  // XCDs of an MI355X
 
 __device__ __forceinline__ float gelu_tanh_g(float v) {
   const float k0 = 0.7978845608028654f;  // sqrt(2 / pi)
@@ -43,165 +69,318 @@ struct GemmArgs {
   const float* res;
   const float* ln_g;   // LayerNorm of the x rows (NULL: none)
   const float* ln_b;
-  const float* stats;  // [M][2] mean, 1/std of the x rows (with LN; NULL: computed here)
   float ln_eps;
   int M, N, K;
   int act;    // 0 none, 1 GELU (tanh form)
   int split;  // > 0: column n goes to segment n / split of a [N/split][M][split] output
+  int mt;     // row tiles (set at launch)
 };
 
-// Row mean and 1/sqrt(var + eps) (population variance, jax_backend.py:78-82),
-// one wavefront per row; sums of the values shifted by the row's first
-// element.
-__global__ __launch_bounds__(256) void k_rowstats(float* __restrict__ stats,
-                                                  const float* __restrict__ x, int M, int K,
-                                                  float eps) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
-  if (row >= M) return;
-  const float* xr = x + (size_t)row * K;
+// Mean and 1/sqrt(var + eps) of a row of K values (population variance,
+// jax_backend.py:78-82), by one wavefront: sums of the values shifted by the
+// row's first element.
+__device__ __forceinline__ float2 row_stats(const float* xr, int K, float eps, int lane) {
   const float c = xr[0];
   float s = 0.f, q = 0.f;
-  for (int j = l; j < K; j += 64) {
-    const float v = xr[j] - c;
-    s += v;
-    q += v * v;
+  for (int j = 4 * lane; j < K; j += 256) {  // K % 4 == 0
+    const f32x4 v = *reinterpret_cast<const f32x4*>(xr + j);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float d = v[t] - c;
+      s += d;
+      q += d * d;
+    }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     s += __shfl_xor(s, o);
     q += __shfl_xor(q, o);
   }
-  if (l == 0) {
-    const float ms = s / K;
-    stats[(size_t)row * 2] = c + ms;
-    stats[(size_t)row * 2 + 1] = 1.f / sqrtf(fmaxf(q / K - ms * ms, 0.f) + eps);
+  const float ms = s / K;
+  return make_float2(c + ms, 1.f / sqrtf(fmaxf(q / K - ms * ms, 0.f) + eps));
+}
+
+// y = LayerNorm(x) of M rows, one wavefront per row (the second pass over a
+// row reads it from the caches). Normalised once here, the rows cost the GEMM
+// nothing; normalising them as each column tile splits them took 3 more
+// vector instructions a value and the gamma and beta loads.
+__global__ __launch_bounds__(256) void k_layernorm_rows(float* __restrict__ y,
+                                                        const float* __restrict__ x,
+                                                        const float* __restrict__ g,
+                                                        const float* __restrict__ b, int M, int K,
+                                                        float eps) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= M) return;
+  const float* xr = x + (size_t)row * K;
+  const float2 st = row_stats(xr, K, eps, lane);
+  for (int j = 4 * lane; j < K; j += 256) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(xr + j);
+    const f32x4 gj = *reinterpret_cast<const f32x4*>(g + j);
+    const f32x4 bj = *reinterpret_cast<const f32x4*>(b + j);
+    f32x4 o;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] = (v[t] - st.x) * st.y * gj[t] + bj[t];
+    *reinterpret_cast<f32x4*>(y + (size_t)row * K + j) = o;
   }
 }
 
-template <bool LN>
-__global__ __launch_bounds__(kThreads) void k_gemm(GemmArgs a) {
-  __shared__ __attribute__((aligned(16))) float sA[kBM * kSP];
-  __shared__ __attribute__((aligned(16))) float sB[kBN * kSP];
+// 16-byte chunk `chunk` (8 k) of row `row` in an LDS plane (element offset).
+__device__ __forceinline__ int plane_at(int row, int chunk) {
+  return row * kBK + ((chunk ^ ((row >> 2) & 3)) * 8);
+}
+
+// Two fp32 values as three words of two bf16 parts each (the first in the
+// low half). The parts of a value that is not finite, or that rounds to
+// infinity in bf16, hold a NaN or infinities of both signs.
+__device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+  const float rx = x - bf16w_lo(h), ry = y - bf16w_hi(h);
+  m = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{rx, ry}, bf16x2));
+  l = __builtin_bit_cast(uint32_t, __builtin_convertvector(
+                                       f32x2{rx - bf16w_lo(m), ry - bf16w_hi(m)}, bf16x2));
+}
+
+// 16 bytes at byte offset off of a buffer; zeros where off passes its end.
+__device__ __forceinline__ f32x4 buf_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_of(const float* p, long floats) {
+  // 32-bit sizes: callers pass at most a tile's rows
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)(uint32_t)(floats * 4),
+                                           0x00020000 /* raw 32-bit data */);
+}
+
+// One workgroup: BM x BN outputs, (BM / WM) * (BN / WN) wavefronts of WM x
+// WN. LN: LayerNorm of the x values as they are split (calls without the
+// workspace for k_layernorm_rows).
+template <int BM, int BN, int WM, int WN, bool LN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a) {
+  constexpr int NT = (BM / WM) * (BN / WN) * 64;
+  constexpr int TI = WM / 32, TJ = WN / 32;          // 32 x 32 tiles of a wavefront
+  constexpr int QA = BM * 8 / NT, QB = BN * 8 / NT;  // quads of x and of w per thread and step
+  static_assert(QA * NT == BM * 8 && QB * NT == BN * 8, "staging shape");
+  constexpr int PA = BM * kBK, PB = BN * kBK;  // elements of a plane
+  // [stage][x planes h, m, l; w planes h, m, l]
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 3 * (PA + PB)];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, hf = lane >> 5;
-  const int wm = wave >> 1, wn = wave & 1;  // the wavefront's 64 x 64 quadrant
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
+  const int wm = wave / (BN / WN), wn = wave % (BN / WN);
+  const int xcd = blockIdx.x % kXCD, rest = blockIdx.x / kXCD;
+  const int m0 = (rest % a.mt) * BM, n0 = ((rest / a.mt) * kXCD + xcd) * BN;
+  if (n0 >= a.N) return;
 
-  // staging: float4 e = tid + 256 u of a 128 x 32 tile is row e / 8, k 4 (e % 8)
-  f32x4 ra[kLoads], rb[kLoads];
-  float mu[LN ? kLoads : 1], rs[LN ? kLoads : 1];
+  float mu[LN ? QA : 1], rs[LN ? QA : 1];
   if constexpr (LN) {
-    __shared__ float sstat[LN ? kBM : 1][2];
-    const float* st = a.stats;
-    if (st == nullptr) {
-      // row statistics of this tile's rows, one wavefront per row (shifted by
-      // the row's first element, as k_rowstats)
-      for (int rr = wave; rr < kBM; rr += kThreads / 64) {
-        const float* xr = a.x + (size_t)min(m0 + rr, a.M - 1) * a.K;
-        const float c0 = xr[0];
+    // statistics of this tile's rows, one wavefront per row
+    __shared__ float sstat[BM][2];
+    for (int rr = wave; rr < BM; rr += NT / 64) {
+      const float2 ms = row_stats(a.x + (size_t)min(m0 + rr, a.M - 1) * a.K, a.K, a.ln_eps, lane);
+      if (lane == 0) {
+        sstat[rr][0] = ms.x;
+        sstat[rr][1] = ms.y;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < QA; ++u) {
+      mu[u] = sstat[(tid + NT * u) >> 3][0];
+      rs[u] = sstat[(tid + NT * u) >> 3][1];
+    }
+  }
+
+  // Quad e = tid + NT u of a step is row e / 8, k 4 (e % 8) .. + 3 (a
+  // wavefront's load covers 8 whole 128-byte rows), through buffer descriptors
+  // over the tile's rows, so that rows past M or N and k past K read zeros and
+  // no load sits behind a branch (K % 4 == 0: a quad lies wholly inside or
+  // past K).
+  const __amdgpu_buffer_rsrc_t bx =
+      buf_of(a.x + (size_t)m0 * a.K, (long)min(BM, a.M - m0) * a.K);
+  const __amdgpu_buffer_rsrc_t bw =
+      buf_of(a.wt + (size_t)n0 * a.K, (long)min(BN, a.N - n0) * a.K);
+  const __amdgpu_buffer_rsrc_t bg = buf_of(LN ? a.ln_g : a.x, LN ? a.K : 0);
+  const __amdgpu_buffer_rsrc_t bb = buf_of(LN ? a.ln_b : a.x, LN ? a.K : 0);
+  // (NT % 8 == 0: every quad of a thread has the same k)
+  const int kq = 4 * (tid & 7);
+  uint32_t offx[QA], offw[QB];
+#pragma unroll
+  for (int u = 0; u < QA; ++u) offx[u] = (uint32_t)((tid + NT * u) >> 3) * a.K * 4u;
+#pragma unroll
+  for (int u = 0; u < QB; ++u) offw[u] = (uint32_t)((tid + NT * u) >> 3) * a.K * 4u;
+  struct Set {
+    f32x4 q[QA + QB], g[1], b[1];
+  } set[2];
+  auto load_quad = [&](Set& r, int k0, int u) {  // quad u: of x, then of w
+    const int kk = k0 + kq;
+    const uint32_t past = kk < a.K ? 0u : 0xffffffffu;
+    r.q[u] = u < QA ? buf_load(bx, (offx[u < QA ? u : 0] + kk * 4u) | past)
+                    : buf_load(bw, (offw[u < QA ? 0 : u - QA] + kk * 4u) | past);
+  };
+  auto load_ln = [&](Set& r, int k0) {
+    if constexpr (LN) {
+      r.g[0] = buf_load(bg, (uint32_t)(k0 + kq) * 4u);
+      r.b[0] = buf_load(bb, (uint32_t)(k0 + kq) * 4u);
+    }
+  };
+  u32x2 ph, pm, pl;  // the parts of the quad being split
+  // Pair i of a step: half i % 2 of quad i / 2; the second half stores the
+  // quad and loads its successor.
+  auto split_pair = [&](Set& r, int stage, int i, int k_next) {
+    const int u = i >> 1, q = i & 1;
+    float x = r.q[u][2 * q], y = r.q[u][2 * q + 1];
+    if constexpr (LN) {
+      if (u < QA) {
+        const float mm = mu[u < QA ? u : 0], ss = rs[u < QA ? u : 0];
+        x = (x - mm) * ss * r.g[0][2 * q] + r.b[0][2 * q];
+        y = (y - mm) * ss * r.g[0][2 * q + 1] + r.b[0][2 * q + 1];
+      }
+    }
+    uint32_t h, m, l;
+    split2(x, y, h, m, l);
+    ph[q] = h;
+    pm[q] = m;
+    pl[q] = l;
+    if (q == 1) {
+      const int e = tid + NT * (u < QA ? u : u - QA);
+      uint16_t* p = lds + stage * 3 * (PA + PB) + (u < QA ? 0 : 3 * PA) +
+                    plane_at(e >> 3, (e & 7) >> 1) + 4 * (e & 1);
+      const int stride = u < QA ? PA : PB;
+      *reinterpret_cast<u32x2*>(p) = ph;
+      *reinterpret_cast<u32x2*>(p + stride) = pm;
+      *reinterpret_cast<u32x2*>(p + 2 * stride) = pl;
+      load_quad(r, k_next, u);
+      if (u == QA - 1) load_ln(r, k_next);
+    }
+  };
+
+  f32x16 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = f32x16{};
+
+  const int steps = (a.K + kBK - 1) / kBK;
+  constexpr int NP = 2 * (QA + QB);  // pairs of a thread and step
+  // step 0 goes to LDS at once; steps 1 and 2 wait in registers
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+#pragma unroll
+    for (int u = 0; u < QA + QB; ++u) load_quad(set[f], f * kBK, u);
+    load_ln(set[f], f * kBK);
+    __builtin_amdgcn_sched_barrier(0);  // the sets' loads in the loop's order
+  }
+#pragma unroll
+  for (int i = 0; i < NP; ++i) split_pair(set[0], 0, i, 2 * kBK);
+  __syncthreads();
+
+  // Operands of one 16-k block: the two blocks of a step have a register set
+  // each, so the second one's reads are issued before the products of the
+  // first.
+  struct Frag {
+    bf16x8 x[TI][3], w[TJ][3];
+  } fr[2];
+  auto read_block = [&](int stage, int ks) {
+    const uint16_t* base = lds + stage * 3 * (PA + PB);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+        fr[ks].x[i][p] = *reinterpret_cast<const bf16x8*>(
+            base + p * PA + plane_at(wm * WM + i * 32 + c, 2 * ks + hf));
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+        fr[ks].w[j][p] = *reinterpret_cast<const bf16x8*>(
+            base + 3 * PA + p * PB + plane_at(wn * WN + j * 32 + c, 2 * ks + hf));
+    }
+  };
+
+  // Step s (s % 2 == F): its products from LDS stage F, and between them the
+  // split of step s + 1 into the other stage and the loads of step s + 3.
+  auto step = [&](auto fc, int s) {
+    constexpr int F = decltype(fc)::value, W = F ^ 1;
+    constexpr int SLOTS = kBK / 16 * 6;
+    read_block(F, 0);
+#pragma unroll
+    for (int ks = 0; ks < kBK / 16; ++ks) {
+      if (ks == 0) read_block(F, 1);
+      // the six products, small ones first; planes 0 h, 1 m, 2 l
+      constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int t = 0; t < 6; ++t) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                fr[ks].x[i][px[t]], fr[ks].w[j][pw[t]], acc[i][j], 0, 0, 0);
+        const int slot = ks * 6 + t;
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+          if (i * SLOTS / NP == slot) split_pair(set[W], W, i, (s + 3) * kBK);
+      }
+    }
+    __syncthreads();  // stage F is read, stage W written
+  };
+  // steps in pairs without a branch between them (a step past K adds zeros)
+  for (int s = 0; s < steps; s += 2) {
+    step(std::integral_constant<int, 0>{}, s);
+    step(std::integral_constant<int, 1>{}, s + 1);
+  }
+
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+  if (__ballot(bad) != 0ull) {
+    // an infinity among the operands (or a result that is none): the
+    // wavefront's outputs again with fp32 products
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = f32x16{};
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const int m = min(m0 + wm * WM + i * 32 + c, a.M - 1);
+      const float* xr = a.x + (size_t)m * a.K;
+      float mi = 0.f, ri = 0.f;
+      if constexpr (LN) {  // one row per lane here, as row_stats
         float sm = 0.f, sq = 0.f;
-        for (int j = lane; j < a.K; j += 64) {
-          const float v = xr[j] - c0;
+        for (int k = 0; k < a.K; ++k) {
+          const float v = xr[k] - xr[0];
           sm += v;
           sq += v * v;
         }
+        const float ms = sm / a.K;
+        mi = xr[0] + ms;
+        ri = 1.f / sqrtf(fmaxf(sq / a.K - ms * ms, 0.f) + a.ln_eps);
+      }
+      for (int k = hf; k < a.K; k += 2) {
+        float x = xr[k];
+        if constexpr (LN) x = (x - mi) * ri * a.ln_g[k] + a.ln_b[k];
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-          sm += __shfl_xor(sm, o);
-          sq += __shfl_xor(sq, o);
+        for (int j = 0; j < TJ; ++j) {
+          const int n = min(n0 + wn * WN + j * 32 + c, a.N - 1);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, a.wt[(size_t)n * a.K + k],
+                                                           acc[i][j], 0, 0, 0);
         }
-        if (lane == 0) {
-          const float ms = sm / a.K;
-          sstat[rr][0] = c0 + ms;
-          sstat[rr][1] = 1.f / sqrtf(fmaxf(sq / a.K - ms * ms, 0.f) + a.ln_eps);
-        }
       }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < kLoads; ++u) {
-      const int r = (tid + kThreads * u) >> 3;
-      const int m = min(m0 + r, a.M - 1);
-      mu[u] = st ? st[(size_t)m * 2] : sstat[r][0];
-      rs[u] = st ? st[(size_t)m * 2 + 1] : sstat[r][1];
-    }
-  }
-  // Global loads read clamped, in-bounds addresses; values past K are
-  // zeroed afterwards (K % 4 == 0, so a float4 lies wholly inside or past K).
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < kLoads; ++u) {
-      const int e = tid + kThreads * u, r = e >> 3, kk = k0 + 4 * (e & 7);
-      const int kc = min(kk, a.K - 4);
-      ra[u] = *reinterpret_cast<const f32x4*>(a.x + (size_t)min(m0 + r, a.M - 1) * a.K + kc);
-      rb[u] = *reinterpret_cast<const f32x4*>(a.wt + (size_t)min(n0 + r, a.N - 1) * a.K + kc);
-    }
-  };
-  auto store_tile = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < kLoads; ++u) {
-      const int e = tid + kThreads * u, r = e >> 3, kq = 4 * (e & 7);
-      const bool kin = k0 + kq < a.K;
-      f32x4 va = ra[u], vb = rb[u];
-      if constexpr (LN) {
-        const int kc = min(k0 + kq, a.K - 4);
-        const f32x4 g = *reinterpret_cast<const f32x4*>(a.ln_g + kc);
-        const f32x4 bb = *reinterpret_cast<const f32x4*>(a.ln_b + kc);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) va[t] = (va[t] - mu[u]) * rs[u] * g[t] + bb[t];
-      }
-      if (!kin) {
-        va = f32x4{0.f, 0.f, 0.f, 0.f};
-        vb = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      *reinterpret_cast<f32x4*>(sA + r * kSP + kq) = va;
-      *reinterpret_cast<f32x4*>(sB + r * kSP + kq) = vb;
-    }
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-
-  const int steps = (a.K + kBK - 1) / kBK;
-  load_tile(0);
-  for (int s = 0; s < steps; ++s) {
-    __syncthreads();  // every wavefront is done with the previous step's tiles
-    store_tile(s * kBK);
-    __syncthreads();
-    if (s + 1 < steps) load_tile((s + 1) * kBK);  // in flight during the products
-#pragma unroll
-    for (int g = 0; g < kBK / 8; ++g) {
-      f32x4 fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[i] = *reinterpret_cast<const f32x4*>(sA + (wm * 64 + i * 32 + c) * kSP + 8 * g + 4 * hf);
-        fb[i] = *reinterpret_cast<const f32x4*>(sB + (wn * 64 + i * 32 + c) * kSP + 8 * g + 4 * hf);
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[j][t], acc[i][j], 0, 0, 0);
     }
   }
 
-  // acc[i][j][r]: row m0 + 64 wm + 32 i + 8 (r/4) + 4 hf + r%4, column n0 + 64 wn + 32 j + c
+  // acc[i][j][r]: row m0 + WM wm + 32 i + 8 (r/4) + 4 hf + r%4, column n0 + WN wn + 32 j + c
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = n0 + wn * 64 + j * 32 + c;
+  for (int j = 0; j < TJ; ++j) {
+    const int n = n0 + wn * WN + j * 32 + c;
     if (n >= a.N) continue;
     const float bv = a.bias ? a.bias[n] : 0.f;
     const int seg = a.split > 0 ? n / a.split : 0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
+        const int m = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
         if (m >= a.M) continue;
         const size_t o = a.split > 0 ? ((size_t)seg * a.M + m) * a.split + (n - seg * a.split)
                                      : (size_t)m * a.N + n;
@@ -213,27 +392,51 @@ __global__ __launch_bounds__(kThreads) void k_gemm(GemmArgs a) {
   }
 }
 
+template <int BM, int BN, int WM, int WN, bool LN = false>
+int launch_gemm(GemmArgs a, hipStream_t s) {
+  a.mt = (a.M + BM - 1) / BM;
+  const long nt = ((a.N + BN - 1) / BN + kXCD - 1) / kXCD * kXCD;
+  SKV_REQUIRE(nt * a.mt < (1L << 31), SKV_E_UNSUPPORTED, "skv_linear: M=%d too large", a.M);
+  hipLaunchKernelGGL((k_gemm<BM, BN, WM, WN, LN>), dim3((unsigned)(nt * a.mt)),
+                     dim3((BM / WM) * (BN / WN) * 64), 0, s, a);
+  return check_launch("skv_linear");
+}
+
 }  // namespace
 
-// skv_linear's path for calls of more than 64 rows (model_ops.hip). stats
-// (may be NULL) holds M * 2 floats for the LayerNorm row statistics.
+// skv_linear's path for calls of more than 64 rows (model_ops.hip). norm
+// (may be NULL) holds M * K floats for the normalised rows of a LayerNorm
+// call.
 int gemm_linear(float* y, const float* x, const float* w_t, const float* bias,
                 const float* residual, const float* ln_gamma, const float* ln_beta, float ln_eps,
-                int M, int N, int K, int activation, int split_cols, float* stats,
+                int M, int N, int K, int activation, int split_cols, float* norm,
                 hipStream_t s) {
-  const bool ln = ln_gamma != nullptr;
-  SKV_REQUIRE((M + kBM - 1) / kBM <= 65535, SKV_E_UNSUPPORTED, "skv_linear: M=%d too large", M);
-  if (ln && stats) {
-    hipLaunchKernelGGL(k_rowstats, dim3((M + 3) / 4), dim3(256), 0, s, stats, x, M, K, ln_eps);
+  GemmArgs a{y, x, w_t, bias, residual, ln_gamma, ln_beta, ln_eps, M, N, K, activation,
+             split_cols, 0};
+  SKV_REQUIRE((long)256 * K * 4 < (1L << 32), SKV_E_UNSUPPORTED,
+              "skv_linear: K=%d too large for a tile's buffer", K);
+  if (ln_gamma != nullptr) {
+    if (norm == nullptr) return launch_gemm<64, 64, 32, 32, true>(a, s);
+    hipLaunchKernelGGL(k_layernorm_rows, dim3((M + 3) / 4), dim3(256), 0, s, norm, x, ln_gamma,
+                       ln_beta, M, K, ln_eps);
     const int rc = check_launch("skv_linear");
     if (rc) return rc;
+    a.x = norm;
+    a.ln_g = a.ln_b = nullptr;
   }
-  GemmArgs a{y, x, w_t, bias, residual, ln_gamma, ln_beta, ln ? stats : nullptr, ln_eps,
-             M, N, K, activation, split_cols};
-  const dim3 grid((N + kBN - 1) / kBN, (M + kBM - 1) / kBM);
-  if (ln) hipLaunchKernelGGL(k_gemm<true>, grid, dim3(kThreads), 0, s, a);
-  else hipLaunchKernelGGL(k_gemm<false>, grid, dim3(kThreads), 0, s, a);
-  return check_launch("skv_linear");
+  // Tiles by how they fill the chip's 256 CUs (measured on MI355X, us):
+  //  - 256 x 128 where there are more than two rounds of them: the fewest
+  //    values split per product (2048 x 50304 x 768: 853, 128 x 64 955, 64 x
+  //    64 1128). With fewer, its long workgroups leave CUs idle (2048 x 2304 x
+  //    768: 70 against 63; 2048 x 768 x 3072: 172 against 79).
+  //  - 64 x 64 where 128 x 64 would not reach half the CUs (644 x 768 x 768:
+  //    18.7 against 20.1; 111 x 640 x 2560: 48 against 53).
+  //  - else 128 x 64 in 8 wavefronts of 32 x 32 (2048 x 768 x 768: 23.5,
+  //    64 x 64 27.7, 256 x 128 53; 644 x 2304 x 768: 29, 64 x 64 34).
+  const auto tiles = [&](long bm, long bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  if (tiles(256, 128) > 2 * 256) return launch_gemm<256, 128, 64, 64>(a, s);
+  if (tiles(128, 64) < 128) return launch_gemm<64, 64, 32, 32>(a, s);
+  return launch_gemm<128, 64, 32, 32>(a, s);
 }
 
 }  // namespace skv

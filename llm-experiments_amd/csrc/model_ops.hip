@@ -1232,8 +1232,9 @@ extern "C" int skv_layernorm(float* y, const float* x, const float* gamma, const
 
 extern "C" size_t skv_linear_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  // the GEMM path (more than one 64-row tile): LayerNorm row statistics
-  if (M > kLinRowsPerBlock) return kLinCntBytes + (size_t)M * 2 * sizeof(float);
+  // the GEMM path (more than one 64-row tile): the normalised rows of a
+  // LayerNorm call
+  if (M > kLinRowsPerBlock) return kLinCntBytes + (size_t)M * K * sizeof(float);
   // the skinny kernel's split and the LN path's k_linear split (either may
   // run for these sizes), after the counters
   const size_t sk = M <= 16 && skinny_steps(K) > 0 ? skinny_ws_bytes(N, skinny_splits(M, N, K)) : 0;
@@ -1257,10 +1258,11 @@ extern "C" int skv_linear(float* y, const float* x, const float* w_t, const floa
   // Many rows (a prompt's prefill): the tiled GEMM, bound by the products
   // rather than by the weight stream.
   if (M > kLinRowsPerBlock) {
-    const bool room = ws != nullptr && ws_bytes >= kLinCntBytes + (size_t)M * 2 * sizeof(float);
-    float* stats = room ? reinterpret_cast<float*>(static_cast<char*>(ws) + kLinCntBytes) : nullptr;
+    const bool room = ws != nullptr && ((uintptr_t)ws & 15) == 0 &&
+                      ws_bytes >= kLinCntBytes + (size_t)M * K * sizeof(float);
+    float* norm = room ? reinterpret_cast<float*>(static_cast<char*>(ws) + kLinCntBytes) : nullptr;
     return gemm_linear(y, x, w_t, bias, residual, ln_gamma, ln_beta, ln_eps, M, N, K, activation,
-                       split_cols, stats, (hipStream_t)stream);
+                       split_cols, norm, (hipStream_t)stream);
   }
   // One row tile over many columns (the tied logits): k_linear_wide.
   {

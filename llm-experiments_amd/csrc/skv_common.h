@@ -223,11 +223,12 @@ int fbwd_wide(float* dq, float* dk, float* dv, const float* q, const float* k, c
               const float* o, const float* L, const float* M, const float* dout, float* delta,
               int B, int N, int H, int D, float scale, int DP, int mode, hipStream_t s);
 
-// skv_linear over more than 64 rows: the tiled MFMA GEMM (gemm.hip). stats:
-// M * 2 floats of workspace, used when ln_gamma is set.
+// skv_linear over more than 64 rows: the tiled MFMA GEMM (gemm.hip). norm:
+// M * K floats of workspace (16-byte aligned, or NULL), used when ln_gamma is
+// set.
 int gemm_linear(float* y, const float* x, const float* w_t, const float* bias,
                 const float* residual, const float* ln_gamma, const float* ln_beta, float ln_eps,
-                int M, int N, int K, int activation, int split_cols, float* stats,
+                int M, int N, int K, int activation, int split_cols, float* norm,
                 hipStream_t s);
 }  // namespace skv
 
