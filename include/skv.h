@@ -230,8 +230,8 @@ size_t skv_prefill_workspace_bytes(int B, int C, int H_q, int D, int n_splits);
  * reference's largest flash_attn_max_head_dim is 256, gpu_device.py:468-471);
  * G = H_q / H_kv in {1, 2, 4, 8}; split over the prefix by n_splits; out, q,
  * the caches and ws 16-byte aligned.
- * fp32 cache: q and out fp32, every product in fp32 (v_mfma_f32_32x32x2_f32,
- * the kernel of skv_flash_fwd); D from 1 to 256, any G; n_splits and the
+ * fp32 cache: q and out fp32, every product with fp32 accuracy (the kernels
+ * of skv_flash_fwd); D from 1 to 256, any G; n_splits and the
  * workspace are not used.
  */
 int skv_prefill_attn(void* out, const void* q, const void* k_cache, const void* v_cache,
@@ -524,7 +524,9 @@ int skv_next_embed(float* x, int32_t* ids, int32_t* seq, const int32_t* argmax_p
  * D from 1 to 256 (the reference's flash_attn_max_head_dim is 128 by
  * default, gpu_types.py:93, and at most 256, gpu_device.py:468-471): the
  * kernel runs at D padded to a multiple of 16 up to 128, to 192 or 256
- * past it, with zeros past D. Products on v_mfma_f32_32x32x2_f32 (fp32).
+ * past it, with zeros past D. Products have fp32 accuracy: up to D = 128 each
+ * is six partial products of operands split into three bf16 parts, past it
+ * v_mfma_f32_32x32x2_f32.
  */
 int skv_flash_fwd(float* out, float* L, float* M, const float* q, const float* k, const float* v,
                   int B, int N, int H, int D, float scale, skv_stream_t stream);
@@ -557,8 +559,8 @@ size_t skv_flash_bwd_fast_workspace_bytes(int B, int N, int H, int D);
  * 128 the head dim is padded to 192 or 256 and the kernels, which keep two
  * 32-row operands and an accumulator of the head dim per wavefront, spill
  * part of them to scratch: correct, but far below the narrow shapes' rate.
- * Products run on v_mfma_f32_32x32x2_f32 (fp32); no atomics, so results are
- * bitwise reproducible. Two forms, by the workspace: with
+ * Products as skv_flash_fwd's; no atomics, so results are bitwise
+ * reproducible. Two forms, by the workspace: with
  * skv_flash_bwd_workspace_bytes, dQ recomputes S and dP (seven products);
  * with skv_flash_bwd_fast_workspace_bytes (D <= 64), the dK/dV
  * kernel writes dS and dQ is formed from it (five products, dS written and

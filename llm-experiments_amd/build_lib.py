@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libskv.so")
 SOURCES = ["skv_api.hip", "append.hip", "decode_attn.hip", "decode_attn_generic.hip",
            "decode_attn_generic_paged.hip", "decode_gqa_mfma.hip",
            "decode_direct.hip", "prefill_attn.hip", "model_ops.hip", "gemm.hip",
-           "sample.hip", "flash_fp32.hip", "flash_fp32.hip:wide_bwd", "bpe_tokenizer.cpp"]
+           "sample.hip", "flash_split.hip", "flash_fp32.hip", "flash_fp32.hip:wide_bwd", "bpe_tokenizer.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -25,7 +25,7 @@ HIPCC_FLAGS = [
     "-std=c++17",
     "-fPIC",
     "-shared",
-    # packed fp32 (v_pk_*_f32) is kept off for all device code on this pool
+    # packed fp32 (v_pk_*_f32) is kept off for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
@@ -40,6 +40,7 @@ def hipcc() -> str:
 # ordinary VGPRs (gfx950 MFMAs take either register file); the default
 # heuristic put them in AGPRs and copied them back and forth every step.
 SOURCE_FLAGS = {"flash_fp32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                "flash_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                 # the flash backward past a head dim of 128: the same source as its own
                 # translation unit, accumulators free to live in AGPRs
                 "flash_fp32.hip:wide_bwd": ["-DSKV_FLASH_WIDE_BWD=1"]}

@@ -1,8 +1,9 @@
-// Causal FlashAttention in fp32 on gfx950: the forward with its row
-// statistics (skv_flash_fwd, also the fp32-cache path of skv_prefill_attn)
-// and the backward (skv_flash_bwd), on v_mfma_f32_32x32x2_f32 (fp32
-// products, fp32 accumulation). The notes below describe the backward; the
-// forward reuses its tiling.
+// Causal FlashAttention in fp32 on gfx950: the entry points of the forward
+// with its row statistics (skv_flash_fwd, also the fp32-cache path of
+// skv_prefill_attn) and of the backward (skv_flash_bwd), and the kernels past a
+// head dim of 128, on v_mfma_f32_32x32x2_f32 (fp32 products, fp32
+// accumulation); up to 128 the kernels are those of flash_split.hip. The notes
+// below describe the backward; the forward reuses its tiling.
 //
 // Reference: simple-llm/src/gpu/gpu_kernels.py:2038-2455 (stage 1, one pass
 // per Q block writing partial dK/dV into a workspace; stage 2, their sum) and
@@ -21,12 +22,9 @@
 //   k_fbwd_dkv  one workgroup per (128 keys, b, h). Per 32-query piece:
 //               S = Q K^T and dP = dO V^T, then dV += P^T dO, dK += dS^T Q.
 // Each of the 4 waves owns 32 rows. Its row operands (Q and dO, or K and V)
-// stay in registers for the whole call (up to a head dim of 64, k_fbwd_dkv
-// keeps V in LDS instead); the other side is staged through LDS 64 rows at a
-// time, the next rows' global loads issued a step ahead, into registers, or,
-// where the kernel runs more wavefronts per SIMD (D <= 64: two for
-// k_fbwd_dkv, three for k_fbwd_dq and the forward), at the top of each step.
-// Work past the causal diagonal is skipped per wave.
+// stay in registers for the whole call; the other side is staged through LDS
+// 64 rows at a time, the next rows' global loads issued a step ahead, into
+// registers. Work past the causal diagonal is skipped per wave.
 //
 // v_mfma_f32_32x32x2_f32 lane layout (lane l, c = l % 32, hf = l / 32):
 //   A (32 x 2): A[c][hf]   B (2 x 32): B[hf][c]
@@ -36,44 +34,22 @@
 // each lane reads 4 consecutive d with one 16-byte load per 4 steps. A
 // C-layout tile is then directly the A or B operand of the next product,
 // k-step (q, t) taking row 8q + 4hf + t.
-#include "skv_common.h"
+#include "flash_args.h"
 
 namespace skv {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef flash_f32x4 f32x4;
 
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
 constexpr int kRows = 32 * kWaves;  // rows (queries or keys) of one workgroup
 constexpr int kCols = 64;           // rows of the other side staged per step
 
-struct FbwdArgs {
-  const float* q;
-  const float* k;
-  const float* v;
-  const float* o;
-  const float* dout;
-  const float* L;
-  const float* M;
-  float* dq;
-  float* dk;
-  float* dv;
-  float* delta;  // [B, N, H] row deltas Dl, written by k_fbwd_dq (or k_fbwd_delta)
-  float* ds;     // dS in 32 x 32 tiles (see ds_tile), written by k_fbwd_dkv<.., true> for k_fbwd_dq_ds
-  int N, H, BH, n_blocks;
-  int D;  // head dim (the padded size is the kernel's template D)
-  float scale, sl2;  // scale and scale * log2(e)
-};
-
 __device__ __forceinline__ f32x16 mfma(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
-
-// 2^x on v_exp_f32 (results below 2^-126 flush toward 0, which no
-// probability here needs).
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Element offset of row n of head h in batch b of a [B, N, H, D] tensor.
 __device__ __forceinline__ size_t row_off(int b, int n, int N, int H, int h, int D) {
@@ -81,44 +57,10 @@ __device__ __forceinline__ size_t row_off(int b, int n, int N, int H, int h, int
 }
 
 // Head dims: the kernels run on the head dim padded to DP, a multiple of 16
-// (two 8-element k groups per row fragment, whole float4 LDS stores). MODE
-// 0: D == DP (16, 32, 64, 128), 16-byte vectors throughout; MODE 1: D < DP
-// with D % 4 == 0 (float4 loads, groups past D read as zeros); MODE 2: any
-// other D (element loads). Padded elements are zeros in every operand that
+// (two 8-element k groups per row fragment, whole float4 LDS stores), in the
+// load modes of flash_shape. Padded elements are zeros in every operand that
 // is contracted over d, and the output rows they produce are never stored,
 // so results equal the unpadded computation.
-// Four consecutive elements c..c+3 of a row with D elements, zeros past D.
-template <int MODE>
-__device__ __forceinline__ f32x4 load4m(const float* row, int c, int D) {
-  if constexpr (MODE == 0) {
-    return *reinterpret_cast<const f32x4*>(row + c);
-  } else if constexpr (MODE == 1) {
-    const bool ok = c < D;  // D % 4 == 0: the group lies wholly inside or past D
-    const f32x4 x = *reinterpret_cast<const f32x4*>(row + (ok ? c : 0));
-    return ok ? x : f32x4{0.f, 0.f, 0.f, 0.f};
-  } else {
-    f32x4 x;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const bool ok = c + t < D;
-      const float v = row[ok ? c + t : 0];
-      x[t] = ok ? v : 0.f;
-    }
-    return x;
-  }
-}
-
-// Stores the elements c..c+3 of y that lie inside a row of D elements.
-template <int MODE>
-__device__ __forceinline__ void store4m(float* row, int c, int D, const f32x4& y) {
-  if constexpr (MODE == 2) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (c + t < D) row[c + t] = y[t];
-  } else {
-    if (c < D) *reinterpret_cast<f32x4*>(row + c) = y;
-  }
-}
 
 // 64 rows x D of two tensors, global -> registers -> LDS (row stride D + 4
 // floats: 16-byte aligned rows, and 16-byte reads of 16 consecutive rows hit
@@ -166,7 +108,7 @@ struct Stage {
 
 // dQ and the row deltas; rank 0 = the last query block (the most keys).
 template <int D, int MODE>
-__global__ __launch_bounds__(kThreads, D <= 64 ? 3 : 1) void k_fbwd_dq(FbwdArgs a) {
+__global__ __launch_bounds__(kThreads, 1) void k_fbwd_dq(FbwdArgs a) {
   constexpr int G = D / 8;             // 16-byte pairs of a row fragment
   constexpr int DT = (D + 31) / 32;    // 32-row tiles of dQ^T
   constexpr int SP = Stage<D, MODE>::SP;
@@ -222,14 +164,12 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 3 : 1) void k_fbwd_dq(FbwdArgs 
   const float* kh = a.k + row_off(b, 0, N, H, h, RS);
   const float* vh = a.v + row_off(b, 0, N, H, h, RS);
   Stage<D, MODE> st;
-  constexpr bool PF = D > 64;  // the next rows a step ahead, in registers
-  if (PF) st.load(kh, vh, 0, N, rs, RS);
+  st.load(kh, vh, 0, N, rs, RS);
   for (int j = 0; j < steps; ++j) {
-    if (!PF) st.load(kh, vh, j * kCols, N, rs, RS);
     __syncthreads();
     st.store(sK, sV);
     __syncthreads();
-    if (PF && j + 1 < steps) st.load(kh, vh, (j + 1) * kCols, N, rs, RS);
+    if (j + 1 < steps) st.load(kh, vh, (j + 1) * kCols, N, rs, RS);
 #pragma unroll
     for (int sub = 0; sub < kCols / 32; ++sub) {
       const int key0 = j * kCols + sub * 32;
@@ -291,31 +231,12 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 3 : 1) void k_fbwd_dq(FbwdArgs 
   }
 }
 
-// dS of the five-product backward in 32 x 32 tiles: tile (query block qb, key
-// block kb) of (b, h) holds 32 rows of 32 floats, row = query qb*32 + i, and
-// within a row key kb*32 + 8 qq + 4 hf + t at position 16 hf + 4 qq + t: the
-// order in which lane (query i, half hf) of k_fbwd_dq_ds takes the keys as
-// k-steps, so that lane reads 64 contiguous bytes and a wavefront a whole
-// 4 KB tile.
-__device__ __forceinline__ float* ds_tile(const FbwdArgs& a, int bh, int qb, int kb) {
-  const int nt = (a.N + 31) >> 5;
-  return a.ds + (((size_t)bh * nt + qb) * nt + kb) * 1024;
-}
-__device__ __forceinline__ int ds_key_pos(int c) {  // key c of a block: 8 qq + 4 hf + t
-  return 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
-}
-
-// dK and dV; rank 0 = key block 0 (the most queries). Up to a head dim of
-// 64 the workgroup's V rows wait in LDS rather than registers, so that two
-// workgroups fit a CU (two wavefronts per SIMD).
-template <int D>
-constexpr bool fbwd_v_in_lds() { return D <= 64; }
-template <int D, int MODE, bool DSO = false>  // DSO: also write dS (a.ds) for k_fbwd_dq_ds
-__global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_dkv(FbwdArgs a) {
+// dK and dV; rank 0 = key block 0 (the most queries).
+template <int D, int MODE>
+__global__ __launch_bounds__(kThreads, 1) void k_fbwd_dkv(FbwdArgs a) {
   constexpr int G = D / 8;
   constexpr int DT = (D + 31) / 32;
   constexpr int SP = Stage<D, MODE>::SP;
-  constexpr bool VL = fbwd_v_in_lds<D>();
   const int RS = MODE == 0 ? D : a.D;  // the real head dim
   // One LDS object: the arrays sit at fixed offsets from each other, so a
   // lane's addresses into all of them are one register plus immediates (as
@@ -324,12 +245,10 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
     float q[kCols * SP];
     float d[kCols * SP];  // dO
     float m2[kCols], il[kCols], dl[kCols];
-    float v[VL ? kRows * SP : 4];  // the block's V rows
   };
   __shared__ Smem sm;
   float* const sQ = sm.q;
   float* const sD = sm.d;
-  float* const sV = sm.v;
   float* const sM2 = sm.m2;
   float* const sIL = sm.il;
   float* const sDL = sm.dl;
@@ -344,14 +263,12 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
   const int krow = wk0 + c;  // a key past N is masked for every query (query < N <= krow)
   const size_t koff = row_off(b, min(krow, N - 1), N, H, h, RS);
 
-  f32x4 kf[G], vf[VL ? 1 : G];
-  float* vrow = sV + (VL ? (wave * 32 + c) * SP + 4 * hf : 0);  // V fragment g: vrow[8 g ..]
+  f32x4 kf[G], vf[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     const int d0 = 8 * g + 4 * hf;
     kf[g] = load4m<MODE>(a.k + koff, d0, RS);
-    if constexpr (VL) *reinterpret_cast<f32x4*>(vrow + 8 * g) = load4m<MODE>(a.v + koff, d0, RS);
-    else vf[g] = load4m<MODE>(a.v + koff, d0, RS);
+    vf[g] = load4m<MODE>(a.v + koff, d0, RS);
   }
   f32x16 dva[DT], dka[DT];
 #pragma unroll
@@ -359,11 +276,6 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
     dva[dt] = f32x16{};
     dka[dt] = f32x16{};
   }
-  // DSO: this lane's place in the dS tiles of its key block (query block 0;
-  // the query block adds a whole row of tiles): key c, rows 4 hf + ...
-  float* dsw = nullptr;
-  if constexpr (DSO)
-    dsw = ds_tile(a, bh, 0, wk0 >> 5) + ds_key_pos(c) + 128 * hf;
 
   const int j0 = (blk * kRows) / kCols;  // first step holding a query >= the block's first key
   const int steps = (N + kCols - 1) / kCols;
@@ -381,18 +293,12 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
   const size_t rs = (size_t)H * RS;
   const float* qh = a.q + row_off(b, 0, N, H, h, RS);
   const float* dh = a.dout + row_off(b, 0, N, H, h, RS);
-  // With V in LDS (two workgroups a CU) the next rows are loaded at the top
-  // of each step, the other workgroup's products covering the wait; with one
-  // workgroup a CU they are loaded a step ahead, into registers.
-  if (!VL && j0 < steps) {
+  // the next rows a step ahead, in registers
+  if (j0 < steps) {
     st.load(qh, dh, j0 * kCols, N, rs, RS);
     SKV_FB_STATS(j0)
   }
   for (int j = j0; j < steps; ++j) {
-    if (VL) {
-      st.load(qh, dh, j * kCols, N, rs, RS);
-      SKV_FB_STATS(j)
-    }
     __syncthreads();
     st.store(sQ, sD);
     if (threadIdx.x < kCols) {
@@ -401,7 +307,7 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
       sDL[threadIdx.x] = dl;
     }
     __syncthreads();
-    if (!VL && j + 1 < steps) {
+    if (j + 1 < steps) {
       st.load(qh, dh, (j + 1) * kCols, N, rs, RS);
       SKV_FB_STATS(j + 1)
     }
@@ -417,9 +323,7 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
       for (int g = 0; g < G; ++g) {
         const f32x4 qa = *reinterpret_cast<const f32x4*>(qr + 8 * g);
         const f32x4 da = *reinterpret_cast<const f32x4*>(dr + 8 * g);
-        f32x4 vg;
-        if constexpr (VL) vg = *reinterpret_cast<const f32x4*>(vrow + 8 * g);
-        else vg = vf[g];
+        const f32x4 vg = vf[g];
         s = mfma(qa.x, kf[g].x, s);
         dp = mfma(da.x, vg.x, dp);
         s = mfma(qa.y, kf[g].y, s);
@@ -466,26 +370,6 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
           }
         }
       }
-      if constexpr (DSO) {
-        // dS of the piece (query block q0 / 32, key block wk0 / 32) for
-        // k_fbwd_dq_ds, in the order its lanes read: for each slot the 32
-        // lanes of a half write one query's 128-byte tile row
-        if (krow < N) {
-          float* tp = dsw + (size_t)(q0 >> 5) * ((N + 31) >> 5) * 1024;
-          if (q0 + 32 <= N) {  // wave-uniform: every row of the tile exists
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              __builtin_nontemporal_store(ds[r], tp + (8 * (r / 4) + (r % 4)) * 32);
-          } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int qi = 8 * (r / 4) + 4 * hf + (r % 4);  // query q0 + qi
-              if (q0 + qi < N)  // row qi of the tile; streamed past the caches (read once, later)
-                __builtin_nontemporal_store(ds[r], tp + (8 * (r / 4) + (r % 4)) * 32);
-            }
-          }
-        }
-      }
       // dV[key][d] += sum_query P^T[key][query] dO[query][d]; dK likewise with dS and Q
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
@@ -523,22 +407,9 @@ __global__ __launch_bounds__(kThreads, fbwd_v_in_lds<D>() ? 2 : 1) void k_fbwd_d
 }
 
 // ---------------------------------------------------------------------------
-// Forward: causal attention with the forward's row statistics, fp32.
+// Forward past a head dim of 128 (up to it: flash_split.hip): causal attention
+// with the forward's row statistics, fp32.
 // ---------------------------------------------------------------------------
-
-struct FfwdArgs {
-  const float* q;  // [B, C, Hq, D]
-  const float* k;  // [B, T_cap, Hkv, D]
-  const float* v;
-  const int32_t* start;  // per-sequence position of query 0 (NULL: 0)
-  const int32_t* n_new;  // per-sequence valid queries (NULL: C)
-  float* out;            // [B, C, Hq, D]; rows i >= n_new[b] get zeros
-  float* L;              // [B, C, Hq] softmax sums (may be NULL)
-  float* M;              // [B, C, Hq] row maxima of the scaled scores (may be NULL)
-  int C, Hq, Hkv, T_cap, BH, n_blocks;
-  int D;  // head dim (the padded size is the kernel's template D)
-  float sl2;  // scale * log2(e)
-};
 
 // One workgroup per (128 queries, b, query head); rank-major order as in the
 // backward. Each wave owns 32 queries (lane c, both halves): per 32-key piece
@@ -547,7 +418,7 @@ struct FfwdArgs {
 // units), so O and l are rescaled on few pieces; the true maximum is kept
 // beside it for M and the final L.
 template <int D, int MODE>
-__global__ __launch_bounds__(kThreads, D <= 64 ? 3 : 1) void k_flash_fwd(FfwdArgs a) {
+__global__ __launch_bounds__(kThreads, 1) void k_flash_fwd(FfwdArgs a) {
   constexpr int G8 = D / 8;
   constexpr int DT = (D + 31) / 32;
   constexpr int SP = Stage<D, MODE>::SP;
@@ -685,14 +556,6 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 3 : 1) void k_flash_fwd(FfwdArg
   }
 }
 
-// ---------------------------------------------------------------------------
-// The five-product backward (head dims up to 64, a workspace that holds dS):
-// k_fbwd_delta writes the row deltas, k_fbwd_dkv also writes dS = P * (dP -
-// Dl) of every (query, key <= query) piece it forms, and k_fbwd_dq_ds forms
-// dQ = scale * dS K from it, so dQ no longer recomputes S and dP (7 products
-// -> 5, at the cost of writing and reading dS once: B * H * N^2 / 2 floats).
-// ---------------------------------------------------------------------------
-
 // Dl = rowsum(dO * O): 16 lanes per (b, n, h) row, lane i = 2 g + hf holding
 // elements 8 g + 4 hf .. + 3 (coalesced: a row's lanes read its 256 bytes);
 // the sums are taken as k_fbwd_dq takes them (each half's fragments in order
@@ -718,135 +581,8 @@ __global__ __launch_bounds__(256) void k_fbwd_delta(FbwdArgs a, long rows) {
   if (i == 0 && row < rows) a.delta[row] = half[0] + half[1];
 }
 
-// dQ from the stored dS: one workgroup per (128 queries, b, h), rank 0 = the
-// last query block; each wave owns 32 queries. Per 32-key piece the lane of
-// query c loads its dS row's keys 8 qq + 4 hf .. + 3 (the k-steps of the
-// product, as k_fbwd_dq orders them) one piece ahead, and K goes through LDS
-// 64 rows at a time. dS of a key past the query (or past N) is masked by a
-// select: k_fbwd_dkv wrote zeros there only for the pieces it formed.
-template <int D, int MODE>
-__global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds(FbwdArgs a) {
-  constexpr int DT = (D + 31) / 32;
-  constexpr int SP = D + 4;
-  constexpr int C4 = D / 4;
-  constexpr int NV = kCols * C4 / kThreads;  // float4 of K per thread per step
-  const int RS = MODE == 0 ? D : a.D;
-  __shared__ __attribute__((aligned(16))) float sK[kCols * SP];
-
-  const int H = a.H, N = a.N;
-  const int bh = (int)(blockIdx.x % (unsigned)a.BH), rank = (int)(blockIdx.x / (unsigned)a.BH);
-  const int b = bh / H, h = bh % H;
-  const int blk = a.n_blocks - 1 - rank;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = lane & 31, hf = lane >> 5;
-  const int qrow = blk * kRows + wave * 32 + c;
-  const bool qok = qrow < N;
-  const int qr = qok ? qrow : N - 1;
-  const int qlim = qok ? qrow : -1;  // keys <= qlim are unmasked
-  const int qb = blk * 4 + wave;  // the wave's query block
-
-  f32x16 acc[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
-  const int q_last = min(blk * kRows + kRows, N) - 1;
-  const int wq_last = blk * kRows + wave * 32 < N ? min(blk * kRows + wave * 32 + 31, N - 1) : -1;
-  const int steps = q_last / kCols + 1;
-  const size_t rs = (size_t)H * RS;
-  const float* kh = a.k + row_off(b, 0, N, H, h, RS);
-
-  // dS of the piece at key0 for this lane: keys key0 + 8 qq + 4 hf + t, 64
-  // contiguous bytes of the tile, loaded a piece ahead; masked only where it
-  // is used (a select there, not here, so the load is not waited for at once)
-  auto load_ds = [&](int key0, f32x4 (&x)[4]) {
-    const float* tp = ds_tile(a, bh, qb, key0 >> 5) + c * 32 + 16 * hf;
-#pragma unroll
-    for (int qq = 0; qq < 4; ++qq) x[qq] = *reinterpret_cast<const f32x4*>(tp + 4 * qq);
-  };
-  f32x4 cur[4], nxt[4] = {};
-  if (wq_last >= 0) load_ds(0, cur);
-  f32x4 kr[NV];  // the next step's K rows, loaded a step ahead
-  auto load_k = [&](int j) {
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-      const int e = threadIdx.x + kThreads * u;
-      const int n = min(j * kCols + e / C4, N - 1);
-      kr[u] = load4m<MODE>(kh + (size_t)n * rs, 4 * (e % C4), RS);
-    }
-  };
-  load_k(0);
-  for (int j = 0; j < steps; ++j) {
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-      const int e = threadIdx.x + kThreads * u;
-      *reinterpret_cast<f32x4*>(sK + (e / C4) * SP + 4 * (e % C4)) = kr[u];
-    }
-    __syncthreads();
-    if (j + 1 < steps) load_k(j + 1);
-#pragma unroll
-    for (int sub = 0; sub < kCols / 32; ++sub) {
-      const int key0 = j * kCols + sub * 32;
-      if (key0 > wq_last) break;  // wave-uniform: every later key is masked for this wave
-      if (key0 + 32 <= wq_last) load_ds(key0 + 32, nxt);
-      // keys past the query (or past N: entries never written) weigh 0, by a select
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          cur[qq][t] = key0 + 8 * qq + 4 * hf + t <= qlim ? cur[qq][t] : 0.f;
-      // dQ^T[d][query] += sum_key K[key][d] dS^T[key][query]
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const int dcol = dt * 32 + c;
-        const bool dok = (MODE == 0 && D % 32 == 0) || dcol < RS;
-        const float* kc = sK + (sub * 32 + 4 * hf) * SP + (dok ? dcol : RS - 1);
-#pragma unroll
-        for (int qq = 0; qq < 4; ++qq) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const float kv = kc[(8 * qq + t) * SP];
-            acc[dt] = mfma(dok ? kv : 0.f, cur[qq][t], acc[dt]);
-          }
-        }
-      }
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq) cur[qq] = nxt[qq];
-    }
-  }
-  if (qok) {
-    const size_t qoff = row_off(b, qr, N, H, h, RS);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-        const int d0 = dt * 32 + 8 * qq + 4 * hf;
-        const f32x4 y = {acc[dt][4 * qq] * a.scale, acc[dt][4 * qq + 1] * a.scale,
-                         acc[dt][4 * qq + 2] * a.scale, acc[dt][4 * qq + 3] * a.scale};
-        store4m<MODE>(a.dq + qoff, d0, RS, y);
-      }
-    }
-  }
-}
-
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Padded head dim and load mode of a head dim: a multiple of 16 up to 128,
-// then 192 or 256 (the forward only: one wavefront per SIMD holds a 256-wide
-// query row set and its accumulators without spilling; the backward's
-// kernels hold two row operands and an accumulator and stop at 128).
-struct FlashShape {
-  int DP, mode;
-};
-FlashShape flash_shape(int D) {
-  const int DP = D <= 128 ? (D + 15) / 16 * 16 : D <= 192 ? 192 : 256;
-  return {DP, D == DP ? 0 : (D % 4 == 0 ? 1 : 2)};
-}
-
-// Expands X(DP, MODE) for every kernel shape.
-#define SKV_FLASH_SHAPES(X)                                                           \
-  X(16, 0) X(16, 1) X(16, 2) X(32, 0) X(32, 1) X(32, 2) X(48, 0) X(48, 1) X(48, 2)    \
-  X(64, 0) X(64, 1) X(64, 2) X(80, 0) X(80, 1) X(80, 2) X(96, 0) X(96, 1) X(96, 2)    \
-  X(112, 0) X(112, 1) X(112, 2) X(128, 0) X(128, 1) X(128, 2)
 // The shapes past 128 (the forward's here; the backward's in the wide
 // translation unit).
 #define SKV_FLASH_WIDE_SHAPES(X) X(192, 0) X(192, 1) X(192, 2) X(256, 0) X(256, 1) X(256, 2)
@@ -897,34 +633,19 @@ int fbwd_wide(float* dq, float* dk, float* dv, const float* q, const float* k, c
 }
 #else
 namespace {
-int fbwd_launch(const FbwdArgs& a, const FlashShape& fs, hipStream_t s) {
-  const dim3 grid((unsigned)(a.n_blocks * a.BH));
-  SKV_FLASH_SHAPES(SKV_FB)
-  return set_error(SKV_E_UNSUPPORTED, "skv_flash_bwd: no kernel for head_dim %d", a.D);
+// The row deltas of the five-product form.
+int fbwd_deltas(const FbwdArgs& a, long rows, hipStream_t s, const char* fn) {
+  const FlashShape fs = flash_shape(a.D);
+#define SKV_DELTA(DD, MM)                                                          \
+  if (fs.DP == DD && fs.mode == MM)                                                \
+    hipLaunchKernelGGL((k_fbwd_delta<DD, MM>), dim3((unsigned)((rows + 15) / 16)),  \
+                       dim3(256), 0, s, a, rows);
+  SKV_DELTA(16, 0) SKV_DELTA(16, 1) SKV_DELTA(16, 2) SKV_DELTA(32, 0) SKV_DELTA(32, 1)
+  SKV_DELTA(32, 2) SKV_DELTA(48, 0) SKV_DELTA(48, 1) SKV_DELTA(48, 2) SKV_DELTA(64, 0)
+  SKV_DELTA(64, 1) SKV_DELTA(64, 2)
+#undef SKV_DELTA
+  return check_launch(fn);
 }
-
-// The five-product backward (a.ds set): row deltas, dK/dV with dS written,
-// then dQ from dS.
-#define SKV_FB_DS(DD, MM)                                                            \
-  if (fs.DP == DD && fs.mode == MM) {                                                \
-    hipLaunchKernelGGL((k_fbwd_delta<DD, MM>), dim3((unsigned)((rows + 15) / 16)),    \
-                       dim3(256), 0, s, a, rows);                                    \
-    int rc = check_launch("skv_flash_bwd");                                          \
-    if (rc) return rc;                                                               \
-    hipLaunchKernelGGL((k_fbwd_dkv<DD, MM, true>), grid, dim3(kThreads), 0, s, a);   \
-    rc = check_launch("skv_flash_bwd");                                              \
-    if (rc) return rc;                                                               \
-    hipLaunchKernelGGL((k_fbwd_dq_ds<DD, MM>), grid, dim3(kThreads), 0, s, a);       \
-    return check_launch("skv_flash_bwd");                                            \
-  }
-int fbwd_launch_ds(const FbwdArgs& a, const FlashShape& fs, long rows, hipStream_t s) {
-  const dim3 grid((unsigned)(a.n_blocks * a.BH));
-  SKV_FB_DS(16, 0) SKV_FB_DS(16, 1) SKV_FB_DS(16, 2) SKV_FB_DS(32, 0) SKV_FB_DS(32, 1)
-  SKV_FB_DS(32, 2) SKV_FB_DS(48, 0) SKV_FB_DS(48, 1) SKV_FB_DS(48, 2) SKV_FB_DS(64, 0)
-  SKV_FB_DS(64, 1) SKV_FB_DS(64, 2)
-  return set_error(SKV_E_UNSUPPORTED, "skv_flash_bwd: no kernel for head_dim %d", a.D);
-}
-#undef SKV_FB_DS
 
 // Workspace of the five-product backward: the row deltas (256-byte
 // aligned block), then dS; 0 where that path does not apply.
@@ -984,9 +705,10 @@ extern "C" int skv_flash_bwd(float* dq, float* dk, float* dv, const float* q, co
     FbwdArgs ad = a;
     ad.ds = reinterpret_cast<float*>(static_cast<char*>(ws) +
                                      ((size_t)B * N * H * sizeof(float) + 255) / 256 * 256);
-    return fbwd_launch_ds(ad, fs, (long)B * N * H, s);
+    const int rc = fbwd_deltas(ad, (long)B * N * H, s, fn);
+    return rc ? rc : flash_bwd_split(ad, s, fn);
   }
-  return fbwd_launch(a, fs, s);
+  return flash_bwd_split(a, s, fn);
 }
 
 namespace skv {
@@ -1011,9 +733,9 @@ int attn_fwd_f32(float* out, float* L, float* M, const float* q, const float* k,
   SKV_REQUIRE((long)a.n_blocks * a.BH < (1L << 31), SKV_E_UNSUPPORTED, "%s: grid too large", fn);
   const dim3 grid((unsigned)(a.n_blocks * a.BH));
   const FlashShape fs = flash_shape(D);
+  if (fs.DP <= 128) return flash_fwd_split(a, s, fn);
 #define SKV_FF(DD, MM) \
   if (fs.DP == DD && fs.mode == MM) hipLaunchKernelGGL((k_flash_fwd<DD, MM>), grid, dim3(kThreads), 0, s, a);
-  SKV_FLASH_SHAPES(SKV_FF)
   SKV_FLASH_WIDE_SHAPES(SKV_FF)
 #undef SKV_FF
   return check_launch(fn);

@@ -7,23 +7,16 @@
 // (model_ops.hip), which is bound by reading the weights rather than by the
 // products.
 //
-// Products: every fp32 operand is split into three bf16 parts, x = h + m + l
-// (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), 8 significant bits
-// each and the differences exact), and a product takes the six partial
-// products of order 2^-16 and larger, hh + hm + mh + mm + hl + lh, on
-// v_mfma_f32_32x32x16_bf16 with fp32 accumulation; what is left out is below
-// 2^-25 of a product. Six bf16 MFMAs do the work of eight
-// v_mfma_f32_32x32x2_f32 in 192 matrix-core cycles instead of 512, and round
-// the accumulator 6 times per 16 k instead of 8.
+// Products: every fp32 operand is split into three bf16 parts and a product
+// takes six partial products on v_mfma_f32_32x32x16_bf16 (split_bf16.h).
 // Measured on MI355X against the fp32 MFMA form of the same kernel (128 x 128
 // tiles, one LDS stage): 2048 x 50304 x 768 1390 -> 853 us (186 TFLOP/s),
 // 2048 x 3072 x 768 with LayerNorm 137 -> 67 us, 2048 x 768 x 3072 220 -> 79
 // us, 111 x 640 x 2560 192 -> 48 us; error against float64 (relative
 // 2-norm) 5.0e-7 -> 4.2e-7 at K = 768 and 9.9e-7 -> 8.6e-7 at K = 3072.
-// The split is exact for finite values; an infinity (or a value that rounds
-// to one in bf16) gives a NaN in its rows or columns, so a wavefront whose
-// sums are not all finite computes them again on v_mfma_f32_32x32x2_f32, which
-// gives what fp32 products give.
+// A wavefront whose sums are not all finite (an infinity, or a value that
+// rounds to one in bf16, among the operands) computes them again on
+// v_mfma_f32_32x32x2_f32, which gives what fp32 products give.
 //
 // Design: a workgroup computes BM x BN outputs, its wavefronts 64 x 64 or 32
 // x 32 each. K goes in steps of 32: quads of 4 consecutive k are read as fp32
@@ -41,16 +34,13 @@
 // tile (0.5 us a step for 64 x 64).
 #include <type_traits>
 
-#include "skv_common.h"
+#include "split_bf16.h"
 
 namespace skv {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBK = 32;  // k per step
@@ -127,17 +117,6 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(float* __restrict__ y,
 // 16-byte chunk `chunk` (8 k) of row `row` in an LDS plane (element offset).
 __device__ __forceinline__ int plane_at(int row, int chunk) {
   return row * kBK + ((chunk ^ ((row >> 2) & 3)) * 8);
-}
-
-// Two fp32 values as three words of two bf16 parts each (the first in the
-// low half). The parts of a value that is not finite, or that rounds to
-// infinity in bf16, hold a NaN or infinities of both signs.
-__device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
-  const float rx = x - bf16w_lo(h), ry = y - bf16w_hi(h);
-  m = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{rx, ry}, bf16x2));
-  l = __builtin_bit_cast(uint32_t, __builtin_convertvector(
-                                       f32x2{rx - bf16w_lo(m), ry - bf16w_hi(m)}, bf16x2));
 }
 
 // 16 bytes at byte offset off of a buffer; zeros where off passes its end.
@@ -302,8 +281,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
 #pragma unroll
     for (int ks = 0; ks < kBK / 16; ++ks) {
       if (ks == 0) read_block(F, 1);
-      // the six products, small ones first; planes 0 h, 1 m, 2 l
-      constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+      // the six partial products
 #pragma unroll
       for (int t = 0; t < 6; ++t) {
 #pragma unroll
@@ -311,7 +289,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
 #pragma unroll
           for (int j = 0; j < TJ; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                fr[ks].x[i][px[t]], fr[ks].w[j][pw[t]], acc[i][j], 0, 0, 0);
+                fr[ks].x[i][kSplitA[t]], fr[ks].w[j][kSplitB[t]], acc[i][j], 0, 0, 0);
         const int slot = ks * 6 + t;
 #pragma unroll
         for (int i = 0; i < NP; ++i)

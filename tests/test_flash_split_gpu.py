@@ -1,0 +1,99 @@
+"""The fp32 flash kernels' split products (csrc/flash_split.hip): head dims at
+the edges of the 16- and 32-wide padding with lengths at the edges of a piece
+and a workgroup, and operands that have no finite bf16 parts."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import banner
+from oracle import kv_oracle as ko
+from test_flash_bwd_gpu import flash_bwd
+from test_flash_fwd_gpu import flash_fwd
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-4  # the bar of the fp32 flash tests
+
+
+def _rel(a, b):
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
+
+
+def _dev(x):
+    return torch.from_numpy(np.ascontiguousarray(x, np.float32)).cuda()
+
+
+@pytest.mark.parametrize("N", [31, 33, 128, 161])
+@pytest.mark.parametrize("D", [15, 16, 17, 33, 50, 64, 65, 84, 97, 112, 128])
+def test_edges_match_oracle(gpu_ctx, N, D):
+    banner(f"flash split N={N} D={D}")
+    B, H = 2, 2
+    rng = np.random.default_rng(N + D)
+    Q, K, V, dO = (rng.standard_normal((B * N, H * D)).astype(np.float32) for _ in range(4))
+    O, L, M = ko.flash_attention(Q, K, V, B, N, H, D)
+    o, Ls, Ms = flash_fwd(_dev(Q), _dev(K), _dev(V), B, N, H, D)
+    for got, want in ((o, O), (Ls, L), (Ms, M)):
+        assert _rel(got.cpu().numpy().reshape(-1), np.asarray(want).reshape(-1)) < TOL
+    want = ko.flash_attention_backward(Q, K, V, O, L, M, dO, B, N, H, D)
+    for fast in (False, True):
+        got = flash_bwd(_dev(Q), _dev(K), _dev(V), _dev(O), _dev(L), _dev(M), _dev(dO), B, N, H,
+                        D, fast=fast)
+        for g, w in zip(got, want):
+            assert _rel(g.cpu().numpy(), w) < TOL
+
+
+def _reference(q, k, v, go):
+    """float64 O, dQ, dK, dV of one causal head [N, D], each query over the
+    keys it sees alone."""
+    q, k, v, go = (t.astype(np.float64) for t in (q, k, v, go))
+    o, dq, dk, dv = (np.zeros_like(q) for _ in range(4))
+    sc = 1.0 / np.sqrt(q.shape[1])
+    for i in range(len(q)):
+        s = (k[:i + 1] @ q[i]) * sc
+        e = np.exp(s - s.max())
+        pr = e / e.sum()
+        o[i] = pr @ v[:i + 1]
+        ds = pr * (v[:i + 1] @ go[i] - (go[i] * o[i]).sum())
+        dq[i] = (ds @ k[:i + 1]) * sc
+        dk[:i + 1] += np.outer(ds, q[i]) * sc
+        dv[:i + 1] += np.outer(pr, go[i])
+    return o, dq, dk, dv
+
+
+@pytest.mark.parametrize("D", [48, 64, 128])
+@pytest.mark.parametrize("what,value", [(w, v) for w in ("q", "k", "v", "go")
+                                        for v in (np.inf, -np.inf)]
+                         + [("q", 3.4e38), ("k", -3.4e38)])
+def test_values_without_bf16_parts(gpu_ctx, D, what, value):
+    """One infinite element, or one that rounds to infinity in bf16, at row 40
+    of head 0: values, infinities and NaN as in the plain computation. (Rows 32
+    to 63 share a piece with it, where a masked key weighs 0 times infinity.)"""
+    banner(f"flash split {what}={value} D={D}")
+    N, H = 200, 2
+    rng = np.random.default_rng(D)
+    t = {n: rng.standard_normal((N, H, D)).astype(np.float32) for n in ("q", "k", "v", "go")}
+    if np.isfinite(value):  # what it meets is small, so the scores stay ordinary
+        t["k" if what == "q" else "q"] *= np.float32(1e-38)
+    t[what][40, 0, 5] = value
+    flat = {n: _dev(x.reshape(N, H * D)) for n, x in t.items()}
+    o, L, M = flash_fwd(flat["q"], flat["k"], flat["v"], 1, N, H, D)
+    grads = flash_bwd(flat["q"], flat["k"], flat["v"], o, L, M, flat["go"], 1, N, H, D,
+                      fast=D <= 64)
+    got = [x.cpu().numpy().reshape(N, H, D).astype(np.float64) for x in (o, *grads)]
+    with np.errstate(all="ignore"):
+        want = [_reference(*(t[n][:, h] for n in ("q", "k", "v", "go"))) for h in range(H)]
+    rows = np.r_[0:32, 64:N]
+    for i, name in enumerate(("o", "dq", "dk", "dv")):
+        a, b = got[i][rows, 0], want[0][i][rows]
+        # gradients of 1e-38 or 1e38 values; and rows whose Dl is not finite,
+        # where every masked key of a piece weighs 0 times infinity
+        if name in ("dq", "dk") and (np.isfinite(value) or what in ("k", "v")):
+            continue
+        assert _rel(got[i][:, 1], want[1][i]) < TOL, name  # the other head
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b), err_msg=name)
+        np.testing.assert_array_equal(np.where(np.isinf(a), a, 0), np.where(np.isinf(b), b, 0),
+                                      err_msg=name)
+        fin = np.isfinite(b)
+        assert _rel(np.where(fin, a, 0), np.where(fin, b, 0)) < TOL, name
