@@ -384,9 +384,11 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 // that the dK/dV kernel wrote (the same bits: the partial products are taken
 // in the same order).
 // Measured on MI355X against the fp32 MFMA forms (B, N, H, D; us): 8, 2048, 16,
-// 64: 1520 -> 1160; 2, 1024, 12, 64: 203 -> 164; 2, 2048, 16, 128: 1055 -> 698;
-// 5, 1605, 8, 96: 707 -> 465; 4, 333, 8, 48: 81 -> 60. The largest relative
+// 64: 1520 -> 1110; 2, 1024, 12, 64: 203 -> 138; 2, 2048, 16, 128: 1055 -> 700;
+// 5, 1605, 8, 96: 707 -> 465; 4, 333, 8, 48: 81 -> 51. The largest relative
 // 2-norm error against float64 of dQ, dK and dV at the first: 1.1e-6 -> 8.3e-7.
+// Before P and dS were formed under the products, and with dQ's K 32 rows a
+// step: 1160, 164 and 60 for the first, second and last.
 // ---------------------------------------------------------------------------
 
 // c += A B as mfma_split(b, a, c) orders the partial products of its factors.
@@ -461,14 +463,14 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   // the query block adds a whole row of tiles): key c, rows 4 hf + ...
   float* dsw = nullptr;
   if constexpr (DSO) dsw = ds_tile(a, bh, 0, wk0 >> 5) + ds_key_pos(c) + 128 * hf;
-  auto store_ds = [&](const f32x16& ds, int q0) {
+  auto store_ds = [&](auto interior, const f32x16& ds, int q0) {
     // for each slot the 32 lanes of a half write one query's 128-byte tile
     // row, past the caches (read once, later)
-    if (krow < N) {
+    if (decltype(interior)::value || krow < N) {
       float* tp = dsw + (size_t)(q0 >> 5) * ((N + 31) >> 5) * 1024;
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (q0 + 32 <= N || q0 + 8 * (r / 4) + 4 * hf + (r % 4) < N)
+        if (decltype(interior)::value || q0 + 8 * (r / 4) + 4 * hf + (r % 4) < N)
           __builtin_nontemporal_store(ds[r], tp + (8 * (r / 4) + (r % 4)) * 32);
     }
   };
@@ -488,6 +490,78 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
       dl = a.delta[sr];
     }
   };
+  // One piece. s[r], dp[r]: query q0 + 8(r/4) + 4hf + r%4, key krow. The
+  // vector work stands between products that do not wait for it: P is formed
+  // and split under dP = dO V^T, dS under dV += P^T dO.
+  auto piece = [&](auto interior, int q0) {
+    f32x16 s = f32x16{}, dp = f32x16{};
+    bf16x8 pf[2][3], df[2][3];
+    auto form_p = [&](int half) {
+#pragma unroll
+      for (int qq = 2 * half; qq < 2 * half + 2; ++qq) {
+        const f32x4 m4 = *reinterpret_cast<const f32x4*>(sm.m2 + 8 * qq + 4 * hf);
+        const f32x4 i4 = *reinterpret_cast<const f32x4*>(sm.il + 8 * qq + 4 * hf);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int r = 4 * qq + t, query = q0 + 8 * qq + 4 * hf + t;
+          const float e = fast_exp2(fmaf(s[r], a.sl2, -m4[t])) * i4[t];
+          s[r] = decltype(interior)::value || (krow <= query && query < N) ? e : 0.f;
+        }
+      }
+    };
+    auto form_ds = [&](int half) {
+#pragma unroll
+      for (int qq = 2 * half; qq < 2 * half + 2; ++qq) {
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(sm.dl + 8 * qq + 4 * hf);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) dp[4 * qq + t] = (dp[4 * qq + t] - d4[t]) * s[4 * qq + t];
+      }
+    };
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      bf16x8 qa[3];
+      read_rows<DP, PS>(sm.q, c, kb, hf, qa);
+      s = mfma_split(qa, kf[kb], s);
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      bf16x8 da[3], vf[3];
+      read_rows<DP, PS>(sm.d, c, kb, hf, da);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) vf[p] = sm.v[wave][kb][p][lane];
+      dp = mfma_split(da, vf, dp);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i * KB / 4 == kb) {
+          if (i < 2) form_p(i);
+          else split_tile(s, i - 2, pf[i - 2]);
+        }
+    }
+    // dV[key][d] += sum_query P^T[key][query] dO[query][d]; dK likewise with dS and Q
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        bf16x8 x[3];
+        read_cols<DP, PS>(sm.d, 16 * kk, dt, lane, x);
+        dva[dt] = mfma_split(pf[kk], x, dva[dt]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i * 2 * DT / 4 == kk * DT + dt) {
+            if (i < 2) form_ds(i);
+            else split_tile(dp, i - 2, df[i - 2]);
+          }
+      }
+    if constexpr (DSO) store_ds(interior, dp, q0);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        bf16x8 x[3];
+        read_cols<DP, PS>(sm.q, 16 * kk, dt, lane, x);
+        dka[dt] = mfma_split(df[kk], x, dka[dt]);
+      }
+  };
   if (j0 < pieces) load_piece(j0);
   for (int j = j0; j < pieces; ++j) {
     __syncthreads();
@@ -503,59 +577,10 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
     const int q0 = j * 32;
     // wave-uniform: every query precedes the wave's keys, or the wave has no key
     if (q0 + 31 < wk0 || wk0 >= N) continue;
-    f32x16 s = f32x16{}, dp = f32x16{};
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      bf16x8 qa[3], da[3], vf[3];
-      read_rows<DP, PS>(sm.q, c, kb, hf, qa);
-      read_rows<DP, PS>(sm.d, c, kb, hf, da);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) vf[p] = sm.v[wave][kb][p][lane];
-      s = mfma_split(qa, kf[kb], s);
-      dp = mfma_split(da, vf, dp);
-    }
-    // s[r], dp[r]: query q0 + 8(r/4) + 4hf + r%4, key krow -> P and dS
     // wave-uniform: every key of the wave precedes every query of the piece
     // and every query exists, so no slot is masked
-    const bool interior = q0 >= wk0 + 31 && q0 + 32 <= N;
-#pragma unroll
-    for (int qq = 0; qq < 4; ++qq) {
-      const int ql = 8 * qq + 4 * hf;
-      const f32x4 m4 = *reinterpret_cast<const f32x4*>(sm.m2 + ql);
-      const f32x4 i4 = *reinterpret_cast<const f32x4*>(sm.il + ql);
-      const f32x4 d4 = *reinterpret_cast<const f32x4*>(sm.dl + ql);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int r = 4 * qq + t;
-        s[r] = fast_exp2(fmaf(s[r], a.sl2, -m4[t])) * i4[t];
-        dp[r] -= d4[t];
-      }
-    }
-    if (!interior) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int query = q0 + 8 * (r / 4) + 4 * hf + (r % 4);
-        s[r] = (krow <= query && query < N) ? s[r] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dp[r] *= s[r];
-    if constexpr (DSO) store_ds(dp, q0);
-    // dV[key][d] += sum_query P^T[key][query] dO[query][d]; dK likewise with dS and Q
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 pf[3], df[3];
-      split_tile(s, kk, pf);
-      split_tile(dp, kk, df);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        bf16x8 x[3];
-        read_cols<DP, PS>(sm.d, 16 * kk, dt, lane, x);
-        dva[dt] = mfma_split(pf, x, dva[dt]);
-        read_cols<DP, PS>(sm.q, 16 * kk, dt, lane, x);
-        dka[dt] = mfma_split(df, x, dka[dt]);
-      }
-    }
+    if (q0 >= wk0 + 31 && q0 + 32 <= N) piece(std::true_type{}, q0);
+    else piece(std::false_type{}, q0);
   }
 
   // Sums that are not all finite: the wave's keys again with fp32 products,
@@ -591,7 +616,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
         s[r] = (krow <= query && query < N) ? e : 0.f;
         dp[r] = s[r] * (dp[r] - a.delta[sr]);
       }
-      if constexpr (DSO) store_ds(dp, q0);
+      if constexpr (DSO) store_ds(std::false_type{}, dp, q0);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int dcol = dt * 32 + c;
@@ -787,13 +812,13 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
 }
 
 // dQ from the stored dS: per 32-key piece the lane of query c loads its dS
-// row's keys one piece ahead, and K goes through LDS. dS of a key past the
+// row's keys a step ahead, and K goes through LDS. dS of a key past the
 // query (or past N) is masked by a select: k_fbwd_dkv_split wrote only the
 // pieces it formed.
 template <int D, int MODE>
 __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
   constexpr int DT = (D + 31) / 32;
-  typedef SplitStage<D, MODE, 32> St;
+  typedef SplitStage<D, MODE, 64> St;
   constexpr int DP = St::DP, PS = St::PS, NV = St::NV;
   const int RS = MODE == 0 ? D : a.D;
   __shared__ __attribute__((aligned(16))) uint16_t sK[3 * PS];
@@ -830,48 +855,63 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
       for (int t = 0; t < 4; ++t)
         x[qq][t] = key0 + 8 * qq + 4 * hf + t <= qlim ? x[qq][t] : 0.f;
   };
-  f32x4 cur[4], nxt[4] = {};
-  if (wq_last >= 0) load_ds(0, cur);
+  // 64 keys a step: their dS (two pieces) and K are loaded a step ahead, the
+  // dS into two register sets used in turn.
+  f32x4 ds[2][2][4] = {};
+  auto load_step = [&](int j, f32x4 (&x)[2][4]) {
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+      if (j * 64 + sub * 32 <= wq_last) load_ds(j * 64 + sub * 32, x[sub]);
+  };
+  const int steps = (pieces + 1) / 2;
+  load_step(0, ds[0]);
   St st;
 #pragma unroll
   for (int i = 0; i < NV; ++i) st.load(i, kh, 0, N, rs, RS);
-  for (int j = 0; j < pieces; ++j) {
+  auto step = [&](auto fc, int j) {
+    constexpr int F = decltype(fc)::value;
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < NV; ++i) st.store(i, sK);
     __syncthreads();
-    if (j + 1 < pieces) {
+    if (j + 1 < steps) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i) st.load(i, kh, (j + 1) * 32, N, rs, RS);
+      for (int i = 0; i < NV; ++i) st.load(i, kh, (j + 1) * 64, N, rs, RS);
+      load_step(j + 1, ds[F ^ 1]);
     }
-    const int key0 = j * 32;
-    if (key0 > wq_last) continue;  // wave-uniform: every later key is masked for this wave
-    if (key0 + 32 <= wq_last) load_ds(key0 + 32, nxt);
-    mask_ds(key0, cur);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 f[3];
-      split8(cur[2 * kk], cur[2 * kk + 1], f);
+    for (int sub = 0; sub < 2; ++sub) {
+      const int key0 = j * 64 + sub * 32;
+      if (key0 > wq_last) break;  // wave-uniform: every later key is masked for this wave
+      f32x4 (&cur)[4] = ds[F][sub];
+      mask_ds(key0, cur);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        bf16x8 kt[3];
-        read_cols<DP, PS>(sK, 16 * kk, dt, lane, kt);
-        acc[dt] = mfma_split(kt, f, acc[dt]);
+      for (int kk = 0; kk < 2; ++kk) {
+        bf16x8 f[3];
+        split8(cur[2 * kk], cur[2 * kk + 1], f);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          bf16x8 kt[3];
+          read_cols<DP, PS>(sK, sub * 32 + 16 * kk, dt, lane, kt);
+          acc[dt] = mfma_split(kt, f, acc[dt]);
+        }
       }
     }
-#pragma unroll
-    for (int qq = 0; qq < 4; ++qq) cur[qq] = nxt[qq];
+  };
+  for (int j = 0; j < steps; j += 2) {
+    step(std::integral_constant<int, 0>{}, j);
+    if (j + 1 < steps) step(std::integral_constant<int, 1>{}, j + 1);
   }
   if (dq_bad(acc, qok, hf, RS)) {  // not all finite: the wave again with fp32 products
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
     for (int key0 = 0; key0 <= wq_last; key0 += 32) {
-      load_ds(key0, cur);
-      mask_ds(key0, cur);
-      f32x16 ds;
+      load_ds(key0, ds[0][0]);
+      mask_ds(key0, ds[0][0]);
+      f32x16 x;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) ds[r] = cur[r >> 2][r & 3];
-      dq_piece_f32(acc, ds, kh, key0, N, rs, RS, c, hf);
+      for (int r = 0; r < 16; ++r) x[r] = ds[0][0][r >> 2][r & 3];
+      dq_piece_f32(acc, x, kh, key0, N, rs, RS, c, hf);
     }
   }
   if (qok) store_dq<DT, MODE>(a, acc, row_off(b, qrow, N, H, h, RS), hf, RS);
