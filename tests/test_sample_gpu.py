@@ -240,3 +240,38 @@ def test_split_draws_follow_the_distribution(gpu_ctx):
     freq = np.bincount(tok, minlength=V) / M
     assert np.isin(tok, hot).all()
     assert np.abs(freq - want).max() < 0.03
+
+
+# The short list of a filtered row (rows past 16,384 entries): one entry, as
+# many as it is asked for at most, one more (dense), ties across the cut, and
+# rows so flat that the list overflows (dense).
+@pytest.mark.parametrize("V", [16385, 53248])
+@pytest.mark.parametrize("spread,step,p", [
+    (2.5, 0.0, dict(top_k=1)), (2.5, 0.0, dict(top_k=128, top_p=0.9)),
+    (2.5, 0.0, dict(top_k=129, top_p=0.9)), (2.5, 0.25, dict(top_k=40, top_p=0.8)),
+    (2.5, 0.25, dict(top_k=7, min_p=0.3)), (0.01, 0.0, dict(top_k=16)),
+    (0.5, 0.0, dict(min_p=0.02, top_p=0.9)), (4.0, 0.0, dict(min_p=0.1))])
+def test_short_list_edges(gpu_ctx, V, spread, step, p):
+    p = dict(dict(T=0.9, top_k=0, top_p=1.0, min_p=0.0, pen=1.0, window=8), **p)
+    banner(f"sample short list V={V} spread={spread} step={step} {p}")
+    r = np.random.default_rng(V)
+    logits = (r.standard_normal((2, V)) * spread).astype(np.float32)
+    if step:
+        logits = np.round(logits / step).astype(np.float32) * np.float32(step)  # ties
+    seq = r.integers(0, V, (2, 8)).astype(np.int32)
+    lens = np.array([8, 8])
+    tok, probs = run_sample(logits, seq, lens, seed=9, **p)
+    tok2, _ = run_sample(logits, seq, lens, seed=9, probs=False, **p)
+    np.testing.assert_array_equal(tok, tok2)
+    for m in range(2):
+        want = oracle_row(logits[m], seq[m], 8, **p)
+        amb = top_p_ambiguous(logits[m], seq[m], 8, **p)
+        # entries within float rounding of the min-p threshold may go either way
+        pre = oracle_row(logits[m], seq[m], 8, **dict(p, top_k=0, top_p=1.0, min_p=0.0))
+        amb |= set(np.nonzero(np.abs(pre - p["min_p"] * pre.max()) < 1e-5 * pre.max())[0].tolist())
+        diff = set(np.nonzero((probs[m] > 0) != (want > 0))[0].tolist())
+        assert diff <= amb, f"row {m}: kept sets differ at {sorted(diff)[:10]}"
+        if not diff:
+            keep = want > 0
+            np.testing.assert_allclose(probs[m][keep], want[keep], rtol=1e-4, atol=1e-9)
+        assert probs[m][tok[m]] > 0
