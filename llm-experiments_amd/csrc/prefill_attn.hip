@@ -17,13 +17,15 @@
 //    O^T += V^T P^T needs (accumulator slot r of rows 8kk..8kk+7 is slot j of
 //    k-block kk). Only V needs a transpose, done once per tile while staging
 //    it into LDS.
-//  * Workgroup = 8 wavefronts of 32 query rows (256 rows). A wavefront fits
-//    the 256 registers of two wavefronts per SIMD at D = 128 (148 at D = 64),
-//    so two run on each SIMD and the softmax of one overlaps the MFMAs of
-//    the other. (With 4 wavefronts of 64 rows, each
-//    K/V operand fed two MFMAs, but ~460 registers were live and the
-//    compiler shuttled values between AGPRs and VGPRs on every tile: 11%
-//    slower, measured on MI355X.) K/V tiles of 64 tokens are double
+//  * A wavefront holds 32 query rows. It fits the 256 registers of two
+//    wavefronts per SIMD at D = 128 (148 at D = 64), so two run on each SIMD
+//    and the softmax of one overlaps the MFMAs of the other. (With 4
+//    wavefronts of 64 rows, each K/V operand fed two MFMAs, but ~460
+//    registers were live and the compiler shuttled values between AGPRs and
+//    VGPRs on every tile: 11% slower, measured on MI355X.) A workgroup has 8
+//    wavefronts (256 rows, one workgroup per CU) where equal chunks fill the
+//    card, and 4 (128 rows, two per CU, see tile_waves) elsewhere: a row
+//    gives the same bits in both. K/V tiles of 64 tokens are double
 //    buffered: the global loads of tile t+1 are in flight while tile t is
 //    computed. Grouped-query attention folds the G query heads of a kv
 //    head into the rows (row = query * G + head), so K/V are read once per
@@ -36,7 +38,7 @@
 //    SIMD: each holds twice the queries and accumulators) and 128 KB of
 //    double-buffered K/V tiles.
 //  * Long prefixes are split into n_splits token ranges (split-K, so that
-//    about one workgroup runs per CU); partials (m, l, o[D]) are merged by a
+//    every CU has work); partials (m, l, o[D]) are merged by a
 //    second pass. The query tiles of one (sequence, kv head, split) are laid
 //    out 8 blocks apart so they land on the same XCD together and the second
 //    tile's K/V reads hit that XCD's L2. (A merge by the last split of each
@@ -46,6 +48,7 @@
 //    more than the 12 us merge pass.)
 //  * Rows i >= n_new[b] of the output are written as zeros by the workgroup
 //    that owns them (one split) or by the merge pass.
+#include <cmath>
 #include <type_traits>
 
 #include "skv_common.h"
@@ -57,14 +60,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kWaves = 8;                   // wavefronts per workgroup up to D = 128
+constexpr int kWaves = 8;                   // most wavefronts of a workgroup
 constexpr int kQB = 1;                      // 32-row query blocks per wavefront
-constexpr int kBM = kWaves * kQB * 32;      // query rows per workgroup (256)
-
-// Wavefronts per workgroup at kernel head dim D: 8 (two per SIMD) up to 128;
-// at 256 a wavefront holds twice the queries and accumulators (~310
-// registers), so 4 (one per SIMD, 512 registers each) and 128 query rows.
-constexpr int waves_for(int D) { return D > 128 ? 4 : kWaves; }
+constexpr int kCUs = 256;                   // CUs of an MI355X
 constexpr int kBN = 64;                     // tokens per K/V tile
 constexpr int kXCD = 8;                     // XCDs of an MI355X
 
@@ -160,11 +158,12 @@ __device__ __forceinline__ void store4(void* out, size_t i, int dt, const float 
 // LV = 0: D is the real head dim (64 or 128) and tiles move by LDS DMA.
 // LV = 8 or 1: D is the padded head dim, a.D the real one; tiles move
 // through registers, 16-byte loads (a.D % 8 == 0) or element loads.
-template <int D, int G, int LV>
-__global__ __launch_bounds__(waves_for(D) * 64, 1) void k_prefill_mfma(PrefillArgs a) {
+// W: wavefronts per workgroup (4 at D = 256, where a wavefront holds twice
+// the queries and accumulators, ~310 registers: one per SIMD).
+template <int D, int G, int LV, int W>
+__global__ __launch_bounds__(W * 64, D > 128 ? 1 : 2) void k_prefill_mfma(PrefillArgs a) {
   constexpr int KB = D / 16;  // k-blocks of the QK^T product
   constexpr int DB = D / 32;  // 32-row d blocks of O^T
-  constexpr int W = waves_for(D);
   constexpr int BM = W * kQB * 32;  // query rows of the workgroup
   constexpr bool GEN = LV != 0;
   const int RS = GEN ? a.D : D;  // row stride of q, out and the cache rows
@@ -631,10 +630,9 @@ __global__ __launch_bounds__(256) void k_prefill_merge(PrefillArgs a) {
   }
 }
 
-// Query tiles of a (sequence, kv head) at kernel head dim DK (the plan,
-// which does not know the head dim, counts them at DK = 128).
-int n_query_tiles(int C, int G, int DK = 128) {
-  const int bm = waves_for(DK) * kQB * 32;
+// Query tiles of a (sequence, kv head) for workgroups of this many wavefronts.
+int n_query_tiles(int C, int G, int waves) {
+  const int bm = waves * kQB * 32;
   return (C * G + bm - 1) / bm;
 }
 
@@ -643,6 +641,43 @@ int n_query_tiles(int C, int G, int DK = 128) {
 int kernel_dim(int D) {
   if (D == 64 || D == 128 || D >= 256) return D;
   return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
+}
+
+// How tiles move: 0 = LDS DMA at an exact head dim of 64, 128 or 256 (a
+// 32-wide row is a quarter of a DMA piece's lanes and has no such kernel);
+// 8 = 16-byte register loads; 1 = element loads.
+int load_form(int D) { return kernel_dim(D) == D && D != 32 ? 0 : (D % 8 == 0 ? 8 : 1); }
+
+// Whether a 256-row and a 128-row kernel exist (the latter at two workgroups
+// per CU). The element-load form stages a tile at the cost of its products,
+// so halving the rows that share it is slower (head dim 100, 16 (sequence,
+// head) pairs, 500 queries after 3000: 69 -> 105 us) and it keeps 256 rows.
+bool two_sizes(int D) { return kernel_dim(D) <= 128 && load_form(D) != 1; }
+
+// Wavefronts per workgroup. 256-row workgroups run alone on their CU, so
+// their number is quantized to the CUs and the longest sets the time; two
+// 128-row ones share a CU and its SIMDs, and one left alone runs at more than
+// half the pair's time. With ragged chunks, or equal ones that leave an
+// eighth of a round of CUs idle, 128 rows measured faster on MI355X (bf16,
+// us, 256 -> 128 rows):
+//   6 ragged x 8 kv heads x 4 x 128, <= 333 after <= 1900     64.4 -> 55.7
+//   the same, all 333 after 1900 (288 workgroups of 256)      128 -> 105
+//   8 ragged x 16 x 128, <= 600 after <= 3000                 98.5 -> 77.2
+//   3 x 16 x 128, 640 after 8000 (288 over two splits)         232 -> 151
+//   5 ragged x 16 x 80, <= 900 after <= 3000                   125 -> 102
+//   2 x 4 x 64, 100 after 8000, 8 splits                      28.4 -> 23.5
+// Equal chunks that do fill their rounds share each tile among more rows:
+//   4 x 16 x 128, 512 after 32256, 2 splits                    549 | 582
+//   4 x 8 x 8 x 128, 60 after 30000, 4 splits                  252 | 267
+//   8 x 8 x 2 x 96, 512 after 8000                             285 | 309
+//   8 x 16 x 128, 512 after 2000 / 8000                 88.5, 300 | 89.5, 294
+int tile_waves(int B, int C, int H_kv, int G, int D, int n_splits, bool ragged) {
+  if (kernel_dim(D) > 128) return 4;
+  if (!two_sizes(D)) return kWaves;
+  if (ragged) return 4;
+  const long wg = (long)B * H_kv * n_query_tiles(C, G, kWaves) * n_splits;
+  const long rounds = (wg + kCUs - 1) / kCUs;
+  return 8 * wg >= 7 * rounds * kCUs ? kWaves : 4;
 }
 
 bool dt_ok(int dt) { return dt == SKV_F32 || dt == SKV_BF16; }
@@ -658,21 +693,38 @@ size_t prefill_part_bytes(int B, int C, int H_q, int D, int n_splits) {
 }
 }  // namespace
 
-extern "C" int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits) {
+extern "C" int skv_prefill_plan_dim(int B, int C, int H_q, int H_kv, int D, int max_kv_end,
+                                    int* n_splits) {
   SKV_REQUIRE(n_splits, SKV_E_INVALID, "skv_prefill_plan: null output");
   SKV_REQUIRE(B > 0 && C > 0 && H_q > 0 && H_kv > 0 && max_kv_end > 0 && H_q % H_kv == 0,
               SKV_E_INVALID, "skv_prefill_plan: bad dims (B=%d C=%d H_q=%d H_kv=%d len=%d)", B,
               C, H_q, H_kv, max_kv_end);
-  // About one workgroup per CU (256 on MI355X), and splits of at least four
-  // 64-token tiles.
-  const long wg = (long)B * H_kv * n_query_tiles(C, H_q / H_kv);
-  long ns = (256 + wg - 1) / wg;
-  const long max_ns = (max_kv_end + 4 * kBN - 1) / (4 * kBN);
+  SKV_REQUIRE(D > 0, SKV_E_INVALID, "skv_prefill_plan: bad head dim %d", D);
+  // Splits of 256-row workgroups (128 at a kernel head dim of 256), at most:
+  //  - kernels of one size, one workgroup per CU: what one round of the CUs
+  //    holds, and at least four 64-token tiles a split (2 x 12 x 200, 300
+  //    after 1000: 3 splits 61 us; 4, a second round, 102);
+  //  - kernels of two sizes: enough for seven eighths of the CUs (128-row
+  //    workgroups take the rest; 3 ragged x 12 x 2 x 96, 252 workgroups: 1
+  //    split 81.5 us, 2 splits 106; 7 x 8 x 8 x 128, 224: 118 and 138), and
+  //    sqrt(tokens / 96): a split saves tokens / splits^2 of the walk and
+  //    costs its partials' trip through memory (2 x 4 x 64, 100 after 8000:
+  //    4, 8, 16, 32 splits 30.5, 23.5, 24.4, 34.3 us; 16 x 128, 256 after
+  //    8000: 46.1, 39.6, 46.8 at 4, 8, 16; 12 x 64, 1024 queries: 17.5, 18.0,
+  //    21.4 at 2, 3, 4).
+  const bool two = two_sizes(D);
+  const long wg = (long)B * H_kv * n_query_tiles(C, H_q / H_kv, kernel_dim(D) > 128 ? 4 : kWaves);
+  long ns = two ? (kCUs * 7 / 8 + wg - 1) / wg : kCUs / wg;
+  const long max_ns = two ? (long)sqrt(max_kv_end / 96.0) : (max_kv_end + 4 * kBN - 1) / (4 * kBN);
   if (ns > max_ns) ns = max_ns;
   if (ns > 32) ns = 32;
   if (ns < 1) ns = 1;
   *n_splits = (int)ns;
   return SKV_OK;
+}
+
+extern "C" int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits) {
+  return skv_prefill_plan_dim(B, C, H_q, H_kv, 128, max_kv_end, n_splits);
 }
 
 extern "C" size_t skv_prefill_workspace_bytes(int B, int C, int H_q, int D, int n_splits) {
@@ -754,7 +806,8 @@ int prefill_attn_impl(void* out, const void* q, const void* k_cache, const void*
   a.C = C; a.Hq = H_q; a.Hkv = H_kv; a.T_cap = T_cap;
   a.qscale = scale * LOG2E;
   a.q_dt = q_dt; a.out_dt = out_dt;
-  a.n_qt = n_query_tiles(C, G, DK);
+  const int W = tile_waves(B, C, H_kv, G, D, n_splits, n_new != nullptr);
+  a.n_qt = n_query_tiles(C, G, W);
   a.n_splits = n_splits;
   a.n_groups = B * H_kv * n_splits;
   a.B = B;
@@ -765,19 +818,19 @@ int prefill_attn_impl(void* out, const void* q, const void* k_cache, const void*
   SKV_REQUIRE(blocks < (1L << 31), SKV_E_UNSUPPORTED, "%s: grid too large", fn);
   if (!launch) return SKV_OK;
   hipStream_t s = (hipStream_t)stream;
-  // LV: 0 = LDS DMA at an exact head dim of 64, 128 or 256 (a 32-wide row is a quarter
-  // of a DMA piece's lanes and has no such kernel); 8 = 16-byte register loads; 1 = element
-  // loads
-  const int LV = DK == D && D != 32 ? 0 : (D % 8 == 0 ? 8 : 1);
-#define SKV_PF(DD, GG, LL)                                                                    \
-  if (DK == DD && G == GG && LV == LL)                                                        \
-    hipLaunchKernelGGL((k_prefill_mfma<DD, GG, LL>), dim3((unsigned)blocks),                  \
-                       dim3(waves_for(DD) * 64), 0, s, a);
-#define SKV_PF4(DD, LL) SKV_PF(DD, 1, LL) SKV_PF(DD, 2, LL) SKV_PF(DD, 4, LL) SKV_PF(DD, 8, LL)
-  SKV_PF4(64, 0) SKV_PF4(128, 0) SKV_PF4(256, 0)
-  SKV_PF4(32, 8) SKV_PF4(32, 1) SKV_PF4(64, 8) SKV_PF4(64, 1) SKV_PF4(128, 8) SKV_PF4(128, 1)
-  SKV_PF4(256, 8) SKV_PF4(256, 1)
-#undef SKV_PF4
+  const int LV = load_form(D);
+#define SKV_PF(DD, GG, LL, WW)                                                                \
+  if (DK == DD && G == GG && LV == LL && W == WW)                                             \
+    hipLaunchKernelGGL((k_prefill_mfma<DD, GG, LL, WW>), dim3((unsigned)blocks),              \
+                       dim3(WW * 64), 0, s, a);
+#define SKV_PFG(DD, LL, WW) \
+  SKV_PF(DD, 1, LL, WW) SKV_PF(DD, 2, LL, WW) SKV_PF(DD, 4, LL, WW) SKV_PF(DD, 8, LL, WW)
+  SKV_PFG(64, 0, 4) SKV_PFG(64, 0, 8) SKV_PFG(128, 0, 4) SKV_PFG(128, 0, 8)
+  SKV_PFG(32, 8, 4) SKV_PFG(32, 8, 8) SKV_PFG(64, 8, 4) SKV_PFG(64, 8, 8)
+  SKV_PFG(128, 8, 4) SKV_PFG(128, 8, 8)
+  SKV_PFG(32, 1, 8) SKV_PFG(64, 1, 8) SKV_PFG(128, 1, 8)
+  SKV_PFG(256, 0, 4) SKV_PFG(256, 8, 4) SKV_PFG(256, 1, 4)
+#undef SKV_PFG
 #undef SKV_PF
   int rc = check_launch(fn);
   if (rc) return rc;

@@ -554,7 +554,8 @@ def kv_cache_prefill(ctx: GPUContext, cache: KVCache, layer_idx: int, new_k: tor
     L = _lib.lib()
     stream = _lib.stream_handle(dev)
     cdt, idt = _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype)
-    n_dev = (None if n_new is None else
+    # (counts that are all C are a chunk without counts: no copy to the device)
+    n_dev = (None if n_new is None or int(n_host.min()) == C else
              torch.from_numpy(n_host.astype(np.int32)).to(dev, non_blocking=False))
     n_ptr = n_dev.data_ptr() if n_dev is not None else None
     kc, vc = layer.k_cache.buffer, layer.v_cache.buffer
@@ -563,8 +564,8 @@ def kv_cache_prefill(ctx: GPUContext, cache: KVCache, layer_idx: int, new_k: tor
         if n_splits > 0:
             ns.value = int(n_splits)
         else:
-            _lib.check(L.skv_prefill_plan(B, C, Hq, Hkv, int((start + n_host).max()),
-                                          ctypes.byref(ns)), "skv_prefill_plan")
+            _lib.check(L.skv_prefill_plan_dim(B, C, Hq, Hkv, D, int((start + n_host).max()),
+                                              ctypes.byref(ns)), "skv_prefill_plan_dim")
         need = L.skv_prefill_workspace_bytes(B, C, Hq, D, ns.value)
         ws = _prefill_workspace(ctx, need)
         sc = float(scale) if scale is not None else 1.0 / float(np.sqrt(D))

@@ -294,3 +294,44 @@ def test_fused_prefill_call_equals_the_three_calls(gpu_ctx, cache_dt, n_splits, 
     np.testing.assert_array_equal(l1.numpy(), l0.numpy())
     assert torch.equal(k1, k0) and torch.equal(v1, v0)
     assert torch.equal(o1, o0)  # NaN-filled before: every element written, the same bits
+
+
+@pytest.mark.parametrize("D,G", [(32, 2), (64, 1), (96, 4), (128, 1), (128, 8)])
+@pytest.mark.parametrize("C", [16, 127, 129, 256, 300])
+def test_workgroup_sizes_give_the_same_bits(D, G, C):
+    """Equal chunks that fill the card run 256-row workgroups, the same chunk
+    given with per-sequence counts 128-row ones; a row's products, maxima and
+    sums are taken in the same order in both (a tile past a row's own limit
+    adds exact zeros), so outputs agree in every bit."""
+    from simple_llm_amd import _lib
+    L = _lib.lib()
+    s = torch.cuda.current_stream().cuda_stream
+    rows = (C * G + 255) // 256  # 256-row tiles of a (sequence, kv head)
+    B, Hkv = 4, -(-256 // (4 * rows))  # a full round: at least seven eighths of the CUs
+    Hq, T = Hkv * G, 500 + C
+    gen = torch.Generator(device="cuda").manual_seed(D * 1000 + C)
+    k = torch.randn(B, T, Hkv, D, device="cuda", generator=gen).to(torch.bfloat16)
+    v = torch.randn(B, T, Hkv, D, device="cuda", generator=gen).to(torch.bfloat16)
+    q = torch.randn(B, C, Hq, D, device="cuda", generator=gen)
+    start = torch.tensor([0, 1, 63, 500], dtype=torch.int32, device="cuda")
+    full = torch.full((B,), C, dtype=torch.int32, device="cuda")
+    outs = []
+    for n_splits in (1, 3):
+        need = L.skv_prefill_workspace_bytes(B, C, Hq, D, n_splits)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+        for n_ptr in (None, full.data_ptr()):
+            out = torch.full((B, C, Hq, D), float("nan"), device="cuda")
+            _lib.check(L.skv_prefill_attn(out.data_ptr(), q.data_ptr(), k.data_ptr(),
+                                          v.data_ptr(), start.data_ptr(), n_ptr, B, C, Hq, Hkv,
+                                          D, T, D ** -0.5, n_splits, ws.data_ptr(), ws.numel(),
+                                          _lib.BF16, _lib.F32, _lib.F32, s), "skv_prefill_attn")
+            outs.append(out)
+        assert torch.equal(outs[-2], outs[-1])
+    # and against float64 on the bf16-rounded operands, one head of the last sequence
+    kk, vv = (t[3, :, 0].double().cpu() for t in (k, v))
+    qq = q[3, :, 0].to(torch.bfloat16).double().cpu()
+    sc = qq @ kk.T * D ** -0.5
+    sc.masked_fill_(torch.arange(T)[None] > 500 + torch.arange(C)[:, None], float("-inf"))
+    want = torch.softmax(sc, -1) @ vv
+    for o in outs[1::2]:
+        assert rel_err(o[3, :, 0].double().cpu().numpy(), want.numpy()) < BF16_TOL
