@@ -91,6 +91,11 @@ int skv_append_chunk(void* k_cache, void* v_cache, const void* k_new,
                      int B, int C, int H_kv, int D, int T_cap, int cache_dt,
                      int in_dt, skv_stream_t stream);
 
+/* dst[0 .. n) (device) = src[0 .. n) (host), in stream order; src has been read
+ * when the call returns, and nothing waits. For small arrays: 256 integers a
+ * launch. */
+int skv_upload_i32(int32_t* dst, const int32_t* src /* host */, int n, skv_stream_t stream);
+
 /* lens[b] = min(lens[b] + (n_new ? n_new[b] : n_const), T_cap). */
 int skv_advance(int32_t* lens, const int32_t* n_new, int n_const, int B, int T_cap,
                 skv_stream_t stream);

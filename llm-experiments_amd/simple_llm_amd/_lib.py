@@ -13,6 +13,7 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -34,6 +35,7 @@ _SIGNATURES = {
     "skv_append": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
     "skv_append_paged": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
     "skv_append_chunk": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "skv_upload_i32": (_I, [_P, _P, _I, _P]),
     "skv_advance": (_I, [_P, _P, _I, _I, _I, _P]),
     "skv_decode_plan": (_I, [_I, _I, _I, _I, _I, _I, ctypes.c_longlong, _I, ctypes.POINTER(_I),
                                  ctypes.POINTER(_I)]),
@@ -152,6 +154,24 @@ def stream_handle(device: torch.device | None = None) -> int:
     if _RAW_STREAM is not None and idx is not None and torch.cuda.is_initialized():
         return _RAW_STREAM(idx)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+#: Arrays up to this many integers go to the device as kernel arguments (16
+#: launches); longer ones are copied.
+UPLOAD_MAX = 4096
+
+
+def upload_i32(values: np.ndarray, device: torch.device, stream: int) -> torch.Tensor:
+    """A device int32 tensor of a host array's values, in stream order and
+    without waiting for the stream (skv_upload_i32). The caller uses it on
+    `stream`, torch's current one."""
+    host = np.ascontiguousarray(values, np.int32).reshape(-1)
+    if not 0 < host.size <= UPLOAD_MAX:
+        return torch.from_numpy(host).to(device)
+    out = torch.empty(host.size, dtype=torch.int32, device=device)
+    check(lib().skv_upload_i32(out.data_ptr(), host.ctypes.data, host.size, stream),
+          "skv_upload_i32")
+    return out
 
 
 def ptr(t: torch.Tensor) -> int:

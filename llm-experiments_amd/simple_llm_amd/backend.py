@@ -243,13 +243,13 @@ def sample_token(key, logits, temperature, top_k, top_p, min_p, repetition_penal
         return int(out.item())
     if V > 65536:
         raise ValueError("device sampling supports vocab sizes up to 65536")
-    seq = torch.from_numpy(np.ascontiguousarray(recent.astype(np.int32).reshape(1, -1)
-                                                if n else np.zeros((1, 1), np.int32))).to(dev)
-    lens = torch.full((1,), n, dtype=torch.int32, device=dev)
+    # the recent tokens, then their number (the row's length)
+    seq = _lib.upload_i32(np.append(recent, n) if n else np.zeros(2, np.int32), dev, s)
+    lens_ptr = seq.data_ptr() + max(n, 1) * 4
     wsb = L.skv_sample_workspace_bytes(1, V)
     ws = torch.empty(max(wsb, 8), dtype=torch.uint8, device=dev)
     _lib.check(L.skv_sample(out.data_ptr(), None, lg.data_ptr(), seq.data_ptr(),
-                            max(n, 1), lens.data_ptr(), 1, V, float(temperature), int(top_k),
+                            max(n, 1), lens_ptr, 1, V, float(temperature), int(top_k),
                             float(top_p), float(min_p), float(repetition_penalty), n,
                             _seed_of(key), ws.data_ptr(), wsb, s), "skv_sample")
     return int(out.item())

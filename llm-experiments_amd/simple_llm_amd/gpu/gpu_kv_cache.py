@@ -556,7 +556,7 @@ def kv_cache_prefill(ctx: GPUContext, cache: KVCache, layer_idx: int, new_k: tor
     cdt, idt = _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype)
     # (counts that are all C are a chunk without counts: no copy to the device)
     n_dev = (None if n_new is None or int(n_host.min()) == C else
-             torch.from_numpy(n_host.astype(np.int32)).to(dev, non_blocking=False))
+             _lib.upload_i32(n_host, dev, stream))
     n_ptr = n_dev.data_ptr() if n_dev is not None else None
     kc, vc = layer.k_cache.buffer, layer.v_cache.buffer
     if want_attn:
