@@ -468,6 +468,16 @@ int skv_append_decode_attn_direct(void* out, const void* q, void* k_cache, void*
                                   int in_dtype, int q_dtype, int out_dtype, int n_split, void* ws,
                                   size_t ws_bytes, skv_stream_t stream);
 
+/* skv_append_decode_attn_direct with the fill advance of
+ * skv_append_decode_attn, in the same launch: the last of a sequence's
+ * workgroups to finish moves lens[b] (a fill in [0, T_cap)). ws as above, for
+ * every n_split (at least its block of counters), and B * H + B <= 65536. */
+int skv_append_decode_attn_step(void* out, const void* q, void* k_cache, void* v_cache,
+                                const void* new_k, const void* new_v, int32_t* lens, int B, int H,
+                                int D, int T_cap, float scale, int cache_dtype, int in_dtype,
+                                int q_dtype, int out_dtype, int n_split, void* ws,
+                                size_t ws_bytes, skv_stream_t stream);
+
 /* Workspace of skv_append_decode_attn_direct with n_split parts: a fixed
  * 256 KiB block of arrival counters (B * H <= 65536), then B * H * n_split
  * partials (o[D], m, l); 0 for n_split <= 1. The fixed block lets calls of

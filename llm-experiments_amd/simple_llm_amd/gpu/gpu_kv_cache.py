@@ -252,6 +252,35 @@ def _workspace(ctx: GPUContext, nbytes: int) -> torch.Tensor:
     return ws
 
 
+#: One-launch decode steps (skv_append_decode_attn_step): fewer (sequence,
+#: head) pairs than CUs, and at most this many bytes of K and V a pair. Above
+#: them the split kernels spread the rows better. MI355X, kernels of a call
+#: without the append, split -> one launch, us: 8 x 8 x 64 fp32, <= 2040 tokens
+#: 15.2 -> 10.5 (<= 500: 12.3 -> 6.2); 1 x 16 x 128 bf16, 500 / 2000 / 4000
+#: tokens (0.25 / 1 / 2 MB a pair) 13.1 / 14.2 / 15.8 -> 7.7 / 12.7 / 18.7; 16 x
+#: 12 x 64 bf16, 700: 14.3 -> 10.5; 3 x 2 x 128 fp32, <= 3000: 12.8 -> 23.9; 512
+#: pairs of 64 fp32, <= 2000: 46.2 -> 58.1.
+_STEP_PAIRS = 256
+_STEP_BYTES = 1 << 20
+_STEP_SPLIT = 4
+_STEP_STREAMS = 16
+
+
+def _step_workspace(ctx: GPUContext, stream: int):
+    """The one-launch step's workspace (zero-filled once; its counters are zero
+    between calls) for this stream, of one size for every shape that takes
+    it, or None: under a capture that would own the allocation, or past the
+    streams a context keeps one for."""
+    ws = ctx.step_workspaces.get(stream)
+    if ws is None:
+        if len(ctx.step_workspaces) >= _STEP_STREAMS or torch.cuda.is_current_stream_capturing():
+            return None
+        need = _lib.lib().skv_decode_direct_workspace_bytes(1, _STEP_PAIRS, 128, _STEP_SPLIT)
+        ws = ctx.step_workspaces.setdefault(
+            stream, torch.zeros(need, dtype=torch.uint8, device=ctx.device))
+    return ws
+
+
 _WS_BYTES: dict = {}
 _PLAN_OUT = threading.local()
 
@@ -427,14 +456,29 @@ def kv_cache_append_attend(ctx: GPUContext, cache: KVCache, layer_idx: int, new_
         max_len = top
     elif max_len < top:
         _check_max_len(max_len, after)  # raises
+    L = _lib.lib()
+    D, sc = cache.head_dim, float(scale) if scale is not None else 1.0 / math.sqrt(cache.head_dim)
+    stream = _lib.stream_handle(dev)
+    if (not cache.paged and cache.n_heads == cache.n_kv_heads and D in (64, 128)
+            and cache.batch_size * cache.n_heads < _STEP_PAIRS
+            and 2 * max_len * D * cache.layers[0].k_cache.buffer.element_size() <= _STEP_BYTES):
+        ws = _step_workspace(ctx, stream)
+        if ws is not None:
+            rc = L.skv_append_decode_attn_step(
+                out.data_ptr(), q.data_ptr(), layer.k_cache.buffer.data_ptr(),
+                layer.v_cache.buffer.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
+                layer.lens.data_ptr(), cache.batch_size, cache.n_heads, D, cache.max_seq_len, sc,
+                _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype),
+                _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype), _STEP_SPLIT, ws.data_ptr(),
+                ws.numel(), stream)
+            _lib.check(rc, "skv_append_decode_attn_step")
+            layer.host_lens = after
+            return after.copy()
     # every fill is <= max_len here, so the total needs no clamp
     chunk, nchunks = _decode_plan_span(ctx, cache.batch_size, cache.n_heads, cache.n_kv_heads,
                                        max_len, total, cache.head_dim, cache.dtype)
-    L = _lib.lib()
     need = _decode_ws_bytes(cache.batch_size, cache.n_heads, cache.head_dim, nchunks)
     ws = _workspace(ctx, need)
-    sc = float(scale) if scale is not None else 1.0 / math.sqrt(cache.head_dim)
-    stream = _lib.stream_handle(dev)
     cdt, idt = _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype)
     qdt, odt = _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype)
     kc, vc = layer.k_cache.buffer.data_ptr(), layer.v_cache.buffer.data_ptr()

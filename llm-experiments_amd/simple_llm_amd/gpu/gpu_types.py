@@ -83,6 +83,8 @@ class GPUContext:
     reduction_workspace: Optional[GPUBuffer1D] = None
     # split-K workspaces of decode and prefill attention, grown on demand
     decode_workspace: Optional[torch.Tensor] = None
+    # one-launch decode steps: a zero-filled workspace per stream handle
+    step_workspaces: dict = field(default_factory=dict)
     prefill_workspace: Optional[torch.Tensor] = None
 
 

@@ -21,7 +21,8 @@ libskv.so:
     each sequence's last prompt row only;
   * decode: one token per sequence and step: embedding + position, fused
     q/k/v projection (LayerNorm folded into its reads), the cache append and
-    decode attention in one call (skv_append_decode_attn), output projection
+    decode attention in one call (skv_append_decode_attn, or for few rows of
+    short contexts skv_append_decode_attn_step), output projection
     with residual, MLP (LayerNorm folded in, GELU, residual), tied logits and
     the next token, replayed as one HIP graph.
 The next token is skv_argmax when greedy (temperature 0, the reference's
@@ -387,6 +388,8 @@ class TransformerModel:
         lw_ws, lw_n = bf.lin_ws.data_ptr(), bf.lin_ws.numel()
         lens0 = cache.layers[0].lens.data_ptr()
         nsplit = self.direct_split(B, cache.dtype) if direct else 1
+        # few rows of short contexts: attention, append and advance in one launch
+        one = not direct and self._direct_ok() and B * H < 256
         # up to 16 rows: LayerNorm folded into the weights (skv_linear_folded)
         folded = self._folded() if B <= 16 else None
         if not embedded:
@@ -410,6 +413,12 @@ class TransformerModel:
                                                     cdt, _lib.F32, _lib.F32, _lib.F32, nsplit,
                                                     bf.dir_ws.data_ptr(), bf.dir_ws.numel(), s),
                     "skv_append_decode_attn_direct")
+            elif one:
+                chk(L.skv_append_decode_attn_step(attn, q_ptr, kc, vc, k_ptr, v_ptr,
+                                                  layer.lens.data_ptr(), B, H, D, T, scale, cdt,
+                                                  _lib.F32, _lib.F32, _lib.F32, 4,
+                                                  bf.dir_ws.data_ptr(), bf.dir_ws.numel(), s),
+                    "skv_append_decode_attn_step")
             else:
                 chk(L.skv_append_decode_attn(attn, q_ptr, kc, vc, k_ptr, v_ptr,
                                              layer.lens.data_ptr(), B, H, H, D, T, scale, chunk,
@@ -704,8 +713,9 @@ class Generator:
         # Greedy steps of contexts up to 1024 take the direct attention (one
         # workgroup per sequence and head, no merge pass): the step's append
         # leaves the fill where it was and the next step's next-token kernel
-        # advances it. Sampling keeps the split attention, whose advance gives
-        # skv_sample the fill that includes the step's token.
+        # advances it. Sampling takes the attention that advances the fill
+        # itself (skv_append_decode_attn_step, or the split kernels for larger
+        # batches), which gives skv_sample the fill with the step's token.
         self.direct = bool(direct_attention) and self.greedy and model._direct_ok()
         self.reset()
 

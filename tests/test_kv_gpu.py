@@ -697,6 +697,48 @@ def test_direct_attention_matches_oracle(gpu_ctx, B, H, D, T, dt, n_split):
             assert not ws[:65536 * 4].any()
 
 
+@pytest.mark.parametrize("n_split", [1, 2, 4])
+@pytest.mark.parametrize("B,H,D,T,dt", [(1, 4, 64, 256, "f32"), (1, 1, 128, 33, "bf16"),
+                                         (5, 7, 128, 300, "bf16"), (16, 12, 64, 1024, "f32"),
+                                         (255, 1, 64, 40, "bf16")])
+def test_one_launch_step_matches_the_direct_attention(gpu_ctx, B, H, D, T, dt, n_split):
+    """skv_append_decode_attn_step: skv_append_decode_attn_direct's bits (the
+    same kernel) and skv_append_decode_attn's fills, three calls in a row, over
+    empty, last-free-position, full and retired rows; every counter is zero
+    after each call."""
+    from simple_llm_amd import _lib
+    L = _lib.lib()
+    s = _lib.stream_handle()
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    cdt = _lib.dtype_code(tdt)
+    gen = torch.Generator(device="cuda").manual_seed(B + T)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=gen)  # noqa: E731
+    caches = [[t.clone() for t in (rnd(B, T, H, D).to(tdt), rnd(B, T, H, D).to(tdt))]]
+    caches.append([t.clone() for t in caches[0]])
+    fills = np.random.default_rng(B).integers(0, T, B)
+    for i, f in enumerate([T - 2, 0, T, -1, T - 1][:B]):
+        fills[i] = f
+    fills = fills.astype(np.int32)
+    lens = to_dev(fills, torch.int32)
+    ws = torch.zeros(max(L.skv_decode_direct_workspace_bytes(B, H, D, n_split), 65536 * 4),
+                     dtype=torch.uint8, device="cuda")
+    for _ in range(3):
+        q, kn, vn = rnd(B, H, D), rnd(B, H, D), rnd(B, H, D)
+        outs = [torch.full((B, H, D), float("nan"), device="cuda") for _ in range(2)]
+        before = to_dev(fills, torch.int32)
+        for fn, ln, out, (kc, vc) in ((L.skv_append_decode_attn_direct, before, outs[0], caches[0]),
+                                      (L.skv_append_decode_attn_step, lens, outs[1], caches[1])):
+            _lib.check(fn(out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                          kn.data_ptr(), vn.data_ptr(), ln.data_ptr(), B, H, D, T, D ** -0.5,
+                          cdt, _lib.F32, _lib.F32, _lib.F32, n_split, ws.data_ptr(), ws.numel(),
+                          s), "step")
+            assert not ws[:65536 * 4].any()
+        assert torch.equal(outs[0], outs[1])
+        assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+        fills = np.where((fills >= 0) & (fills < T), fills + 1, fills).astype(np.int32)
+        np.testing.assert_array_equal(lens.cpu().numpy(), fills)
+
+
 def test_direct_attention_split_shapes_share_a_workspace(gpu_ctx):
     """Split calls of different shapes (B x H, head dim, dtype) through one
     zero-filled workspace, interleaved: the arrival counters sit in a fixed
