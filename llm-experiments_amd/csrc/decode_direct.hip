@@ -73,6 +73,11 @@ __device__ __forceinline__ float cache_round(float x) {
   else return x;
 }
 
+// The reference of exponentials under a maximum m: -inf - (-inf) would be NaN
+// where every score so far is -inf (or a row or part has none), and their
+// weights are 0.
+__device__ __forceinline__ float finite_ref(float m) { return m == -INFINITY ? 0.f : m; }
+
 // EPL elements of a cache row at element offset i (16-byte vectors for fp32,
 // 8- or 16-byte for bf16).
 template <typename TC, int EPL>
@@ -144,14 +149,15 @@ __global__ __launch_bounds__(kDirRows * 16 / S) void k_decode_direct(DirectArgs 
       s[j] = t0 + j * R < t_hi ? d : -INFINITY;
       smax = fmaxf(smax, s[j]);
     }
-    const float mn = fmaxf(m, smax);  // finite: token t0 < t_hi is valid
-    const float al = fast_exp2(m - mn);
+    const float mn = fmaxf(m, smax);
+    const float mr = finite_ref(mn);
+    const float al = fast_exp2(m - mr);
     l *= al;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) o[e] *= al;
 #pragma unroll
     for (int j = 0; j < TOK; ++j) {
-      const float w = fast_exp2(s[j] - mn);  // 0 for a masked token
+      const float w = fast_exp2(s[j] - mr);  // 0 for a masked token
       l += w;
 #pragma unroll
       for (int e = 0; e < EPL; ++e) o[e] = fmaf(w, vx[j][e], o[e]);
@@ -179,7 +185,8 @@ __global__ __launch_bounds__(kDirRows * 16 / S) void k_decode_direct(DirectArgs 
     for (int e = 0; e < EPL; ++e) d = fmaf(q[e], nk[e], d);
     d = row16_sum(d);
     const float mn = fmaxf(m, d);
-    const float al = fast_exp2(m - mn), w = fast_exp2(d - mn);  // m = -inf: al = 0
+    const float mr = finite_ref(mn);
+    const float al = fast_exp2(m - mr), w = fast_exp2(d - mr);  // m = -inf: al = 0
     l = l * al + w;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) o[e] = fmaf(w, nv[e], o[e] * al);
@@ -198,12 +205,11 @@ __global__ __launch_bounds__(kDirRows * 16 / S) void k_decode_direct(DirectArgs 
   float M = -INFINITY, LL = 0.f, OO = 0.f;
   if (tid < D) {
     for (int r = 0; r < R; ++r) M = fmaxf(M, s_m[r]);
-    if (M != -INFINITY) {
-      for (int r = 0; r < R; ++r) {
-        const float w = fast_exp2(s_m[r] - M);  // rows with no token: 0
-        LL = fmaf(w, s_l[r], LL);
-        OO = fmaf(w, s_o[r][tid], OO);
-      }
+    const float Mr = finite_ref(M);
+    for (int r = 0; r < R; ++r) {
+      const float w = fast_exp2(s_m[r] - Mr);  // rows with no token: 0
+      LL = fmaf(w, s_l[r], LL);
+      OO = fmaf(w, s_o[r][tid], OO);
     }
   }
   const size_t oi = ((size_t)b * a.H + h) * D + tid;
@@ -251,17 +257,18 @@ __global__ __launch_bounds__(kDirRows * 16 / S) void k_decode_direct(DirectArgs 
     for (int z = 0; z < S; ++z) M = fmaxf(M, pm[z]);
     LL = 0.f;
     OO = 0.f;
-    if (M != -INFINITY) {
+    const float Mr = finite_ref(M);
 #pragma unroll
-      for (int z = 0; z < S; ++z) {  // part order: the bits do not depend on the arrival order
-        const float w = fast_exp2(pm[z] - M);  // parts with no token: 0
-        LL = fmaf(w, pl[z], LL);
-        OO = fmaf(w, po[z], OO);
-      }
+    for (int z = 0; z < S; ++z) {  // part order: the bits do not depend on the arrival order
+      const float w = fast_exp2(pm[z] - Mr);  // parts with no token: 0
+      LL = fmaf(w, pl[z], LL);
+      OO = fmaf(w, po[z], OO);
     }
   }
-  // an empty row (no cached token, no append) gives 0, as the split kernels
-  if (tid < D) store_elem(a.out, oi, a.out_dt, LL > 0.f ? OO / LL : 0.f);
+  // an empty row (no cached token, no append) gives 0, as the split kernels;
+  // a NaN among the scores, or scores all of -inf, give NaN
+  const bool any = Lc > 0 || (a.new_k != nullptr && p >= 0 && p < a.T_cap);
+  if (tid < D) store_elem(a.out, oi, a.out_dt, any ? OO / LL : 0.f);
 }
 
 template <typename TC, int D>

@@ -459,14 +459,14 @@ def kv_cache_append_attend(ctx: GPUContext, cache: KVCache, layer_idx: int, new_
     L = _lib.lib()
     D, sc = cache.head_dim, float(scale) if scale is not None else 1.0 / math.sqrt(cache.head_dim)
     stream = _lib.stream_handle(dev)
+    kc, vc = layer.k_cache.buffer.data_ptr(), layer.v_cache.buffer.data_ptr()
     if (not cache.paged and cache.n_heads == cache.n_kv_heads and D in (64, 128)
-            and cache.batch_size * cache.n_heads < _STEP_PAIRS
-            and 2 * max_len * D * cache.layers[0].k_cache.buffer.element_size() <= _STEP_BYTES):
+            and cache.batch_size * cache.n_heads < _STEP_PAIRS and not (kc | vc) & 15
+            and 2 * max_len * D * layer.k_cache.buffer.element_size() <= _STEP_BYTES):
         ws = _step_workspace(ctx, stream)
         if ws is not None:
             rc = L.skv_append_decode_attn_step(
-                out.data_ptr(), q.data_ptr(), layer.k_cache.buffer.data_ptr(),
-                layer.v_cache.buffer.data_ptr(), new_k.data_ptr(), new_v.data_ptr(),
+                out.data_ptr(), q.data_ptr(), kc, vc, new_k.data_ptr(), new_v.data_ptr(),
                 layer.lens.data_ptr(), cache.batch_size, cache.n_heads, D, cache.max_seq_len, sc,
                 _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype),
                 _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype), _STEP_SPLIT, ws.data_ptr(),
@@ -481,7 +481,6 @@ def kv_cache_append_attend(ctx: GPUContext, cache: KVCache, layer_idx: int, new_
     ws = _workspace(ctx, need)
     cdt, idt = _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype)
     qdt, odt = _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype)
-    kc, vc = layer.k_cache.buffer.data_ptr(), layer.v_cache.buffer.data_ptr()
     if cache.paged:
         rc = L.skv_append_decode_attn_paged(
             out.data_ptr(), q.data_ptr(), kc, vc, new_k.data_ptr(), new_v.data_ptr(),

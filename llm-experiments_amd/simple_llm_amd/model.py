@@ -13,9 +13,9 @@ jax_backend.py:25-33). Generation runs in two phases, all HIP kernels of
 libskv.so:
   * prefill: every prompt (a ragged batch) goes through all layers at once:
     embedding + position of every prompt row, the fused q/k/v projection as
-    a tiled MFMA GEMM (LayerNorm applied as the rows are staged), the chunk
+    a tiled MFMA GEMM (LayerNorm in a pass of its own before it), the chunk
     append into the cache, causal attention over it and the fill advance in
-    one call (skv_append_prefill_attn: the fp32 MFMA kernel for an fp32
+    one call (skv_append_prefill_attn: the fp32 kernels for an fp32
     cache, the bf16 one for a bf16 cache), output projection and MLP as
     GEMMs; then the logits of
     each sequence's last prompt row only;
@@ -389,7 +389,7 @@ class TransformerModel:
         lens0 = cache.layers[0].lens.data_ptr()
         nsplit = self.direct_split(B, cache.dtype) if direct else 1
         # few rows of short contexts: attention, append and advance in one launch
-        one = not direct and self._direct_ok() and B * H < 256
+        one = not direct and self._direct_ok() and T <= 1024 and B * H < 256
         # up to 16 rows: LayerNorm folded into the weights (skv_linear_folded)
         folded = self._folded() if B <= 16 else None
         if not embedded:
@@ -413,7 +413,7 @@ class TransformerModel:
                                                     cdt, _lib.F32, _lib.F32, _lib.F32, nsplit,
                                                     bf.dir_ws.data_ptr(), bf.dir_ws.numel(), s),
                     "skv_append_decode_attn_direct")
-            elif one:
+            elif one and not (kc | vc) & 15:  # (16-byte cache rows)
                 chk(L.skv_append_decode_attn_step(attn, q_ptr, kc, vc, k_ptr, v_ptr,
                                                   layer.lens.data_ptr(), B, H, D, T, scale, cdt,
                                                   _lib.F32, _lib.F32, _lib.F32, 4,

@@ -739,6 +739,47 @@ def test_one_launch_step_matches_the_direct_attention(gpu_ctx, B, H, D, T, dt, n
         np.testing.assert_array_equal(lens.cpu().numpy(), fills)
 
 
+@pytest.mark.parametrize("fill", [0, 5, 70, 300])
+@pytest.mark.parametrize("D", [64, 128])
+def test_one_launch_step_with_scores_that_are_not_finite(gpu_ctx, D, fill):
+    """kv_cache_append_attend over few short rows: a score of -inf has weight 0
+    wherever its token falls (alone in a lane row, the new token), a NaN score
+    makes its row NaN and no other, and a row of -inf scores alone is NaN."""
+    gpu = _gpu()
+    B, H, T = 4, 2, 320
+    cache = gpu.kv_cache_create(gpu_ctx, gpu.KVCacheConfig(B, T, 1, H, D))
+    layer = cache.layers[0]
+    gen = torch.Generator(device="cuda").manual_seed(fill + D)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=gen)  # noqa: E731
+    q, nk, nv = rnd(B, H, D), rnd(B, H, D), rnd(B, H, D)
+    k, v = rnd(B, T, H, D), rnd(B, T, H, D)
+    minus = -torch.sign(q) * float("inf")  # q . minus = -inf
+    if fill:
+        k[0, fill - 1, 0] = minus[0, 0]   # row (0, 0): one cached token out
+        k[1, fill // 2, 1] = float("nan")  # row (1, 1): NaN
+        k[3, :fill, 1] = minus[3, 1]       # row (3, 1): the new token alone is left
+    else:
+        nk[1, 1] = float("nan")
+    nk[2, 0] = minus[2, 0]                # row (2, 0): the new token out
+    layer.k_cache.buffer.copy_(k.reshape(B * T, H * D))
+    layer.v_cache.buffer.copy_(v.reshape(B * T, H * D))
+    layer.lens.fill_(fill)
+    layer.host_lens = np.full(B, fill, np.int64)
+    out = torch.empty(B, H, D, device="cuda")
+    gpu.kv_cache_append_attend(gpu_ctx, cache, 0, nk, nv, q, out)
+    got = out.double().cpu()
+    k[:, fill], v[:, fill] = nk, nv
+    kk, vv, qq = (t.double().cpu() for t in (k[:, :fill + 1], v[:, :fill + 1], q))
+    for b in range(B):
+        for h in range(H):
+            sc = (kk[b, :, h] * qq[b, h]).sum(-1) * D ** -0.5
+            want = torch.softmax(sc, 0) @ vv[b, :, h]
+            if torch.isnan(want).any():
+                assert torch.isnan(got[b, h]).all(), (b, h)
+            else:
+                assert rel_err(got[b, h].numpy(), want.numpy()) < FP32_TOL, (b, h)
+
+
 def test_direct_attention_split_shapes_share_a_workspace(gpu_ctx):
     """Split calls of different shapes (B x H, head dim, dtype) through one
     zero-filled workspace, interleaved: the arrival counters sit in a fixed
