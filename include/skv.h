@@ -207,7 +207,8 @@ int skv_append_decode_attn_paged(void* out, const void* q, void* k_pool, void* v
                                  int in_dt, int q_dt, int out_dt, skv_stream_t stream);
 
 /*
- * Split count for skv_prefill_attn (host-only): about one workgroup per CU.
+ * Split count for skv_prefill_attn (host-only): every CU has work, and a split
+ * saves more than its partials cost.
  * max_kv_end = the largest start[b] + n_new[b] of the call.
  */
 int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits /* host */);

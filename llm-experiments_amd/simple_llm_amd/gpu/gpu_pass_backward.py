@@ -4,8 +4,9 @@ Drop-in for flash_attention_backward of simple-llm/src/gpu/gpu_pass_backward.py:
 same arguments, checks and error messages. The reference runs one stage-1
 pass per Q block, each writing partial dK/dV into grad_K_workspace and
 grad_V_workspace, then a reduce pass (gpu/gpu_kernels.py:2038-2455). Here
-skv_flash_bwd computes dQ and then dK/dV in two MFMA kernels with no
-partials; the caller's workspaces are still required and shape-checked as in
+skv_flash_bwd computes dK/dV and dQ in two MFMA kernels (fp32 products, up to
+head_dim 128 as partial products of operands split into three bf16 parts) with no
+partials of whole gradients; the caller's workspaces are still required and shape-checked as in
 the reference, and the row deltas (batch_size * seq_len * n_heads floats)
 are kept in the first bytes of grad_K_workspace.
 """

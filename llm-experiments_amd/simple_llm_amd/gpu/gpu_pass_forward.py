@@ -5,7 +5,8 @@ Drop-in for flash_attention of simple-llm/src/gpu/gpu_pass_forward.py:497-588:
 same arguments, checks and error messages. The reference's WGSL kernel
 (gpu/gpu_kernels.py:499-770) runs one workgroup per (query block, head,
 sequence) with an online softmax over key blocks; skv_flash_fwd runs the same
-computation on fp32 MFMA tiles and writes O, L (softmax sums) and M (row
+computation on MFMA tiles (fp32 products, up to head_dim 128 as six partial
+products of operands split into three bf16 parts) and writes O, L (softmax sums) and M (row
 maxima of the scaled scores), which flash_attention_backward consumes.
 """
 from __future__ import annotations
