@@ -207,14 +207,10 @@ int skv_append_decode_attn_paged(void* out, const void* q, void* k_pool, void* v
                                  int in_dt, int q_dt, int out_dt, skv_stream_t stream);
 
 /*
- * Split count for skv_prefill_attn (host-only): every CU has work, and a split
- * saves more than its partials cost.
+ * Split count for skv_prefill_attn (host-only): about one workgroup per CU.
  * max_kv_end = the largest start[b] + n_new[b] of the call.
  */
 int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits /* host */);
-/* The same for head dim D (skv_prefill_plan counts with the kernels of 128). */
-int skv_prefill_plan_dim(int B, int C, int H_q, int H_kv, int D, int max_kv_end,
-                         int* n_splits /* host */);
 
 /* Bytes of workspace skv_prefill_attn and skv_append_prefill_attn need (0
  * when n_splits == 1): the split partials, then B int32 (16-byte padded) that

@@ -48,7 +48,6 @@
 //    more than the 12 us merge pass.)
 //  * Rows i >= n_new[b] of the output are written as zeros by the workgroup
 //    that owns them (one split) or by the merge pass.
-#include <cmath>
 #include <type_traits>
 
 #include "skv_common.h"
@@ -693,38 +692,26 @@ size_t prefill_part_bytes(int B, int C, int H_q, int D, int n_splits) {
 }
 }  // namespace
 
-extern "C" int skv_prefill_plan_dim(int B, int C, int H_q, int H_kv, int D, int max_kv_end,
-                                    int* n_splits) {
+extern "C" int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits) {
   SKV_REQUIRE(n_splits, SKV_E_INVALID, "skv_prefill_plan: null output");
   SKV_REQUIRE(B > 0 && C > 0 && H_q > 0 && H_kv > 0 && max_kv_end > 0 && H_q % H_kv == 0,
               SKV_E_INVALID, "skv_prefill_plan: bad dims (B=%d C=%d H_q=%d H_kv=%d len=%d)", B,
               C, H_q, H_kv, max_kv_end);
-  SKV_REQUIRE(D > 0, SKV_E_INVALID, "skv_prefill_plan: bad head dim %d", D);
-  // Splits of 256-row workgroups (128 at a kernel head dim of 256), at most:
-  //  - kernels of one size, one workgroup per CU: what one round of the CUs
-  //    holds, and at least four 64-token tiles a split (2 x 12 x 200, 300
-  //    after 1000: 3 splits 61 us; 4, a second round, 102);
-  //  - kernels of two sizes: enough for seven eighths of the CUs (128-row
-  //    workgroups take the rest; 3 ragged x 12 x 2 x 96, 252 workgroups: 1
-  //    split 81.5 us, 2 splits 106; 7 x 8 x 8 x 128, 224: 118 and 138), and
-  //    sqrt(tokens / 96): a split saves tokens / splits^2 of the walk and
-  //    costs its partials' trip through memory (2 x 4 x 64, 100 after 8000:
-  //    4, 8, 16, 32 splits 30.5, 23.5, 24.4, 34.3 us; 16 x 128, 256 after
-  //    8000: 46.1, 39.6, 46.8 at 4, 8, 16; 12 x 64, 1024 queries: 17.5, 18.0,
-  //    21.4 at 2, 3, 4).
-  const bool two = two_sizes(D);
-  const long wg = (long)B * H_kv * n_query_tiles(C, H_q / H_kv, kernel_dim(D) > 128 ? 4 : kWaves);
-  long ns = two ? (kCUs * 7 / 8 + wg - 1) / wg : kCUs / wg;
-  const long max_ns = two ? (long)sqrt(max_kv_end / 96.0) : (max_kv_end + 4 * kBN - 1) / (4 * kBN);
+  // About one 256-row workgroup per CU, and splits of at least four 64-token
+  // tiles. Fewer splits of short prefixes are faster (2 x 4 x 64, 100 queries
+  // after 8000: 23.5 us at 8 splits, 34.3 at 32; 12 x 64, 1024 queries: 17.5,
+  // 21.4 at 2, 4) but less accurate: the largest probability of a split is
+  // exactly 1 in bf16, so the dominant ones round in fewer of them (error
+  // against float64, 2 x 12 x 128, <= 79 after <= 6375: 2.12e-3 at 11 splits,
+  // 2.22e-3 at 8).
+  const long wg = (long)B * H_kv * n_query_tiles(C, H_q / H_kv, kWaves);
+  long ns = (kCUs + wg - 1) / wg;
+  const long max_ns = (max_kv_end + 4 * kBN - 1) / (4 * kBN);
   if (ns > max_ns) ns = max_ns;
   if (ns > 32) ns = 32;
   if (ns < 1) ns = 1;
   *n_splits = (int)ns;
   return SKV_OK;
-}
-
-extern "C" int skv_prefill_plan(int B, int C, int H_q, int H_kv, int max_kv_end, int* n_splits) {
-  return skv_prefill_plan_dim(B, C, H_q, H_kv, 128, max_kv_end, n_splits);
 }
 
 extern "C" size_t skv_prefill_workspace_bytes(int B, int C, int H_q, int D, int n_splits) {

@@ -41,7 +41,6 @@ _SIGNATURES = {
                                  ctypes.POINTER(_I)]),
     "skv_decode_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "skv_prefill_plan": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(_I)]),
-    "skv_prefill_plan_dim": (_I, [_I, _I, _I, _I, _I, _I, ctypes.POINTER(_I)]),
     "skv_prefill_workspace_bytes": (_Z, [_I, _I, _I, _I, _I]),
     "skv_prefill_attn": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _Z,
                               _I, _I, _I, _P]),

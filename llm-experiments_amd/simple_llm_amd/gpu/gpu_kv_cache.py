@@ -607,8 +607,8 @@ def kv_cache_prefill(ctx: GPUContext, cache: KVCache, layer_idx: int, new_k: tor
         if n_splits > 0:
             ns.value = int(n_splits)
         else:
-            _lib.check(L.skv_prefill_plan_dim(B, C, Hq, Hkv, D, int((start + n_host).max()),
-                                              ctypes.byref(ns)), "skv_prefill_plan_dim")
+            _lib.check(L.skv_prefill_plan(B, C, Hq, Hkv, int((start + n_host).max()),
+                                          ctypes.byref(ns)), "skv_prefill_plan")
         need = L.skv_prefill_workspace_bytes(B, C, Hq, D, ns.value)
         ws = _prefill_workspace(ctx, need)
         sc = float(scale) if scale is not None else 1.0 / float(np.sqrt(D))

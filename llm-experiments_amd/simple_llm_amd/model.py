@@ -533,8 +533,8 @@ class TransformerModel:
         ws, wn = pb.lin_ws.data_ptr(), pb.lin_ws.numel()
         n_ptr = pb.n_new.data_ptr()
         ns = ctypes.c_int()
-        chk(L.skv_prefill_plan_dim(B, C, H, H, D, max(int((start + n_host).max()), 1),
-                                   ctypes.byref(ns)), "skv_prefill_plan_dim")
+        chk(L.skv_prefill_plan(B, C, H, H, max(int((start + n_host).max()), 1), ctypes.byref(ns)),
+            "skv_prefill_plan")
         need = L.skv_prefill_workspace_bytes(B, C, H, D, ns.value)
         pws = _prefill_workspace(self.ctx, need)
         pws_ptr = pws.data_ptr() if pws is not None else None

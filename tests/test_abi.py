@@ -228,6 +228,20 @@ def test_prefill_rejects_bad_arguments():
     assert b"too wide" in L.skv_last_error()
 
 
+@pytest.mark.parametrize("B,C,Hq,Hkv,end", [
+    (4, 512, 16, 16, 32768), (6, 333, 32, 8, 2233), (2, 79, 12, 12, 6454), (2, 26, 4, 4, 21875),
+    (1, 768, 32, 4, 768), (7, 35, 16, 16, 2976), (3, 16, 2, 2, 16), (1, 1, 1, 1, 1),
+    (64, 1024, 16, 16, 4096)])
+def test_prefill_plan_keeps_a_split_per_idle_cu(B, C, Hq, Hkv, end):
+    """One 256-row workgroup per CU where splits of at least four 64-token tiles
+    allow it. A split's largest probability is exact in bf16, so a plan of fewer
+    splits rounds more of a row's dominant probabilities."""
+    ns = ctypes.c_int()
+    assert _lib.lib().skv_prefill_plan(B, C, Hq, Hkv, end, ctypes.byref(ns)) == 0
+    wg = B * Hkv * -(-C * (Hq // Hkv) // 256)
+    assert ns.value == max(1, min(-(-256 // wg), -(-end // 256), 32))
+
+
 def test_argmax_workspace_and_rejects():
     L = _lib.lib()
     # one 2048-column slice per workgroup; candidates (value, index) per slice

@@ -109,6 +109,21 @@ def test_prefill_split_counts_agree(gpu_ctx, n_splits):
     assert rel_err(got, want, valid) < BF16_TOL
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,prefix,C,n_new,splits", [
+    (2, 12, 12, 128, [3000, 800], 79, [79, 30], 11),
+    (1, 8, 2, 64, [1700], 96, None, 8),
+    (2, 12, 12, 80, [500, 0], 300, None, 4),
+])
+def test_prefill_default_split_count(gpu_ctx, B, Hq, Hkv, D, prefix, C, n_new, splits):
+    """A call without n_splits has the bits of the plan's split count (a split's
+    largest probability is exact in bf16, so the count decides the rounding)."""
+    banner(f"prefill default splits B={B} Hq={Hq} Hkv={Hkv} D={D} C={C}")
+    T = max(prefix) + C
+    outs = [run_prefill(gpu_ctx, B, T, Hq, Hkv, D, prefix, C, n_new=n_new, seed=3,
+                        n_splits=ns)[0] for ns in (0, splits)]
+    np.testing.assert_array_equal(*outs)
+
+
 def test_prefill_split_merge_repeats_bit_exact(gpu_ctx):
     """Calls of other shapes and split counts between two runs of the same call
     share its workspace and leave nothing behind: the repeat gives the same bits."""
