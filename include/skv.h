@@ -302,7 +302,8 @@ int skv_layernorm(float* y, const float* x, const float* gamma, const float* bet
  * the counters at zero again; with LayerNorm a second kernel sums it.
  * M > 64 (a prompt's prefill): a tiled MFMA GEMM, each fp32 operand as
  * three bf16 parts and a product as the six partial products of order 2^-16
- * and larger (fp32 accuracy; operands with infinities take fp32 products);
+ * and larger (fp32 accuracy over every finite operand, which is scaled by a
+ * power of two first; operands from 2^104 and infinities take fp32 products);
  * with LayerNorm, ws (16-byte aligned) of skv_linear_workspace_bytes(M, N,
  * K) bytes holds the normalised rows, computed once (without it every column
  * tile normalises its own).
@@ -540,7 +541,8 @@ int skv_next_embed(float* x, int32_t* ids, int32_t* seq, const int32_t* argmax_p
  * default, gpu_types.py:93, and at most 256, gpu_device.py:468-471): the
  * kernel runs at D padded to a multiple of 16 up to 128, to 192 or 256
  * past it, with zeros past D. Products have fp32 accuracy: up to D = 128 each
- * is six partial products of operands split into three bf16 parts, past it
+ * is six partial products of operands split into three bf16 parts (scaled by
+ * a power of two first, so that small operands keep every bit), past it
  * v_mfma_f32_32x32x2_f32.
  */
 int skv_flash_fwd(float* out, float* L, float* M, const float* q, const float* k, const float* v,

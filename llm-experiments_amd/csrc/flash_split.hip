@@ -79,13 +79,14 @@ struct SplitStage {
     const int n = min(row0 + e / C4, n_rows - 1);
     r[u] = load4m<MODE>(t + (uint64_t)(uint32_t)n * rs, 4 * (e % C4), Dr);
   }
-  __device__ __forceinline__ void store(int u, uint16_t* planes) const {
+  __device__ __forceinline__ void store(int u, uint16_t* planes, float scale) const {
     const int e = quad(u), row = e / C4, q = e % C4;
     u32x2 h, m, l;
     uint32_t a, b, c;
-    split2(r[u].x, r[u].y, a, b, c);
+    const f32x4 x = r[u] * scale;
+    split2(x.x, x.y, a, b, c);
     h.x = a; m.x = b; l.x = c;
-    split2(r[u].z, r[u].w, a, b, c);
+    split2(x.z, x.w, a, b, c);
     h.y = a; m.y = b; l.y = c;
     uint16_t* p = planes + swz<DP>(row, q >> 1) + 4 * (q & 1);
     *reinterpret_cast<u32x2*>(p) = h;
@@ -121,7 +122,7 @@ __device__ __forceinline__ void read_cols(const uint16_t* planes, int r0, int db
   }
 }
 
-// 8 consecutive values of a row, split.
+// 8 consecutive scaled values of a row, split.
 __device__ __forceinline__ void split8(const f32x4& x, const f32x4& y, bf16x8 (&f)[3]) {
   u32x4 w[3];
 #pragma unroll
@@ -135,7 +136,7 @@ __device__ __forceinline__ void split8(const f32x4& x, const f32x4& y, bf16x8 (&
   for (int p = 0; p < 3; ++p) f[p] = __builtin_bit_cast(bf16x8, w[p]);
 }
 
-// k-block kk of a C tile as an operand.
+// k-block kk of a (scaled) C tile as an operand.
 __device__ __forceinline__ void split_tile(const f32x16& t, int kk, bf16x8 (&f)[3]) {
   split8(f32x4{t[8 * kk], t[8 * kk + 1], t[8 * kk + 2], t[8 * kk + 3]},
          f32x4{t[8 * kk + 4], t[8 * kk + 5], t[8 * kk + 6], t[8 * kk + 7]}, f);
@@ -207,9 +208,9 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
   float m_run = -INFINITY, m_true = -INFINITY, l = 0.f;
 
   // The online softmax of the piece at key0: s holds its scores in log2 units
-  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query) and gets the
-  // probabilities.
-  auto softmax = [&](f32x16& s, int key0) {
+  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query), times unit's
+  // inverse, and gets the probabilities times p_scale.
+  auto softmax = [&](f32x16& s, int key0, float unit, float p_scale) {
     // A piece wholly at or below the diagonal of a wave whose 32 queries are
     // all valid masks nothing (wave-uniform test).
     float tmax = -INFINITY;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-    tmax = xor32_max(tmax);  // both halves hold the same query
+    tmax = xor32_max(tmax) * unit;  // both halves hold the same query
     m_true = fmaxf(m_true, tmax);
     const bool upd = tmax > m_run + 8.f;  // also true on the first piece with a key
     if (__ballot(upd) != 0ull) {          // wave-uniform branch
@@ -238,16 +239,18 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     const float m_use = m_run == -INFINITY ? 0.f : m_run;  // nothing unmasked yet
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(s[r] - m_use);
+      s[r] = fast_exp2(fmaf(s[r], unit, -m_use));
       l += s[r];
+      s[r] *= p_scale;
     }
   };
 
-  bf16x8 qf[KB][3];  // the query, scaled so that the scores come out in log2 units
+  bf16x8 qf[KB][3];  // the query, so that the scores come out in log2 units
+  const float qs = a.sl2 * kSplitScale;
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb)
-    split8(load4m<MODE>(qp, 16 * kb + 8 * hf, RS) * a.sl2,
-           load4m<MODE>(qp, 16 * kb + 8 * hf + 4, RS) * a.sl2, qf[kb]);
+    split8(load4m<MODE>(qp, 16 * kb + 8 * hf, RS) * qs,
+           load4m<MODE>(qp, 16 * kb + 8 * hf + 4, RS) * qs, qf[kb]);
   St st[2];  // K, V: the piece after the one in LDS
   constexpr int NV = St::NV;
   auto load_quad = [&](int i, int key0) {  // quad i of a piece: of K, then of V
@@ -258,7 +261,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     for (int i = 0; i < 2 * NV; ++i) load_quad(i, 0);
 #pragma unroll
     for (int i = 0; i < 2 * NV; ++i) {
-      st[i / NV].store(i % NV, lds[0] + (i / NV) * 3 * PS);
+      st[i / NV].store(i % NV, lds[0] + (i / NV) * 3 * PS, kSplitScale);
       load_quad(i, 32);
     }
   }
@@ -270,7 +273,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     const uint16_t* const sV = lds[F] + 3 * PS;
     const int key0 = j * 32;
     auto stage_quad = [&](int i) {  // of piece j + 1; its register then takes piece j + 2
-      st[i / NV].store(i % NV, lds[F ^ 1] + (i / NV) * 3 * PS);
+      st[i / NV].store(i % NV, lds[F ^ 1] + (i / NV) * 3 * PS, kSplitScale);
       load_quad(i, key0 + 64);
     };
     if (key0 <= wq_last) {  // wave-uniform: else every key is masked for this wave
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
         for (int i = 0; i < 2 * NV; ++i)
           if (i * KB / (2 * NV) == kb) stage_quad(i);
       }
-      softmax(s, key0);
+      softmax(s, key0, kSplitUnscale, kSplitScale);
       // O^T[d][query] += sum_key V[key][d] P^T[key][query]
       bf16x8 pf[2][3];
       split_tile(s, 0, pf[0]);
@@ -314,9 +317,11 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] += acl[dt];
 
-  // Sums that are not all finite (an infinity or a NaN among the operands):
+  // Sums that are not all finite (an infinity, a NaN or a value too large to
+  // scale among the operands), or a query whose scores all came out as -inf:
   // the wave's queries again with fp32 products, straight from global memory.
-  bool bad = qok && !finite(lt);
+  float unscale = kSplitUnscale;
+  bool bad = qok && !(lt > 0.f && finite(lt));
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -327,6 +332,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     for (int dt = 0; dt < DT; ++dt) acc[dt] = acl[LO ? dt : 0] = f32x16{};
     m_run = m_true = -INFINITY;
     l = 0.f;
+    unscale = 1.f;
     for (int key0 = 0; key0 <= wq_last; key0 += 32) {
       f32x16 s = f32x16{};
       const float* kr = kh + (size_t)min(key0 + c, kv_end - 1) * rs;
@@ -337,7 +343,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
         for (int t = 0; t < 4; ++t) s = mfma_f32(ka[t], qa[t], s);
       }
       s *= a.sl2;
-      softmax(s, key0);
+      softmax(s, key0, 1.f, 1.f);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int dcol = dt * 32 + c;
@@ -354,7 +360,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 
   if (qi >= C) return;
   const size_t orow = ((size_t)b * C + qi) * Hq + h;
-  const float inv = qok ? 1.f / lt : 0.f;  // a valid row saw its own key: lt >= 1
+  const float inv = qok ? 1.f / lt * unscale : 0.f;  // a valid row saw its own key: lt >= 1
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
@@ -390,6 +396,13 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 // Before P and dS were formed under the products, and with dQ's K 32 rows a
 // step: 1160, 164 and 60 for the first, second and last.
 // ---------------------------------------------------------------------------
+
+// The operands are split as 2^16 x here, so that what the chain of products
+// carries, 2^32 for S and dP, 2^48 for dS (of dP and 2^16 P) and 2^64 for dK
+// and dQ, leaves room for large gradients (a sum past the largest float takes
+// the fp32 form); operands below 2^-142 (fp32 subnormals) keep fewer bits.
+constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
+constexpr float kProdScale = 0x1p32f, kDsUnscale = 0x1p-48f, kGradUnscale = 0x1p-64f;
 
 // c += A B as mfma_split(b, a, c) orders the partial products of its factors.
 __device__ __forceinline__ f32x16 mfma_split_swapped(const bf16x8 (&a)[3], const bf16x8 (&b)[3],
@@ -450,9 +463,11 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int d0 = 16 * kb + 8 * hf;
-    split8(load4m<MODE>(a.k + koff, d0, RS), load4m<MODE>(a.k + koff, d0 + 4, RS), kf[kb]);
+    split8(load4m<MODE>(a.k + koff, d0, RS) * kScale,
+           load4m<MODE>(a.k + koff, d0 + 4, RS) * kScale, kf[kb]);
     bf16x8 vf[3];
-    split8(load4m<MODE>(a.v + koff, d0, RS), load4m<MODE>(a.v + koff, d0 + 4, RS), vf);
+    split8(load4m<MODE>(a.v + koff, d0, RS) * kScale,
+           load4m<MODE>(a.v + koff, d0 + 4, RS) * kScale, vf);
 #pragma unroll
     for (int p = 0; p < 3; ++p) sm.v[wave][kb][p][lane] = vf[p];
   }
@@ -463,7 +478,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   // the query block adds a whole row of tiles): key c, rows 4 hf + ...
   float* dsw = nullptr;
   if constexpr (DSO) dsw = ds_tile(a, bh, 0, wk0 >> 5) + ds_key_pos(c) + 128 * hf;
-  auto store_ds = [&](auto interior, const f32x16& ds, int q0) {
+  auto store_ds = [&](auto interior, const f32x16& ds, float unit, int q0) {
     // for each slot the 32 lanes of a half write one query's 128-byte tile
     // row, past the caches (read once, later)
     if (decltype(interior)::value || krow < N) {
@@ -471,7 +486,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (decltype(interior)::value || q0 + 8 * (r / 4) + 4 * hf + (r % 4) < N)
-          __builtin_nontemporal_store(ds[r], tp + (8 * (r / 4) + (r % 4)) * 32);
+          __builtin_nontemporal_store(ds[r] * unit, tp + (8 * (r / 4) + (r % 4)) * 32);
     }
   };
 
@@ -486,13 +501,15 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
     if (threadIdx.x < 32) {  // statistics of query j * 32 + threadIdx.x, clamped
       const size_t sr = (size_t)(b * N + min(j * 32 + (int)threadIdx.x, N - 1)) * H + h;
       m2 = a.M[sr] * LOG2E;
-      il = 1.f / a.L[sr];
-      dl = a.delta[sr];
+      il = 1.f / a.L[sr] * kScale;
+      dl = a.delta[sr] * kProdScale;
     }
   };
+  const float sl2 = a.sl2 * kUnscale;
   // One piece. s[r], dp[r]: query q0 + 8(r/4) + 4hf + r%4, key krow. The
   // vector work stands between products that do not wait for it: P is formed
-  // and split under dP = dO V^T, dS under dV += P^T dO.
+  // and split under dP = dO V^T, dS under dV += P^T dO. S and dP carry 2^32,
+  // P (by il) 2^16 and dS, of P and dP, 2^48.
   auto piece = [&](auto interior, int q0) {
     f32x16 s = f32x16{}, dp = f32x16{};
     bf16x8 pf[2][3], df[2][3];
@@ -504,7 +521,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * qq + t, query = q0 + 8 * qq + 4 * hf + t;
-          const float e = fast_exp2(fmaf(s[r], a.sl2, -m4[t])) * i4[t];
+          const float e = fast_exp2(fmaf(s[r], sl2, -m4[t])) * i4[t];
           s[r] = decltype(interior)::value || (krow <= query && query < N) ? e : 0.f;
         }
       }
@@ -552,7 +569,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
             else split_tile(dp, i - 2, df[i - 2]);
           }
       }
-    if constexpr (DSO) store_ds(interior, dp, q0);
+    if constexpr (DSO) store_ds(interior, dp, kDsUnscale, q0);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -566,7 +583,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   for (int j = j0; j < pieces; ++j) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sm.q : sm.d);
+    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sm.q : sm.d, kScale);
     if (threadIdx.x < 32) {
       sm.m2[threadIdx.x] = m2;
       sm.il[threadIdx.x] = il;
@@ -585,6 +602,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 
   // Sums that are not all finite: the wave's keys again with fp32 products,
   // straight from global memory.
+  float unv = kUnscale, unk = kGradUnscale;
   bool bad = false;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -595,6 +613,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   if (__ballot(bad) != 0ull) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) dva[dt] = dka[dt] = f32x16{};
+    unv = unk = 1.f;
     for (int q0 = wk0; q0 < N; q0 += 32) {
       f32x16 s = f32x16{}, dp = f32x16{};
       const size_t qo = (size_t)min(q0 + c, N - 1) * rs;
@@ -616,7 +635,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
         s[r] = (krow <= query && query < N) ? e : 0.f;
         dp[r] = s[r] * (dp[r] - a.delta[sr]);
       }
-      if constexpr (DSO) store_ds(std::false_type{}, dp, q0);
+      if constexpr (DSO) store_ds(std::false_type{}, dp, 1.f, q0);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int dcol = dt * 32 + c;
@@ -640,8 +659,8 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
       const int key = wk0 + 8 * (r / 4) + 4 * hf + (r % 4);
       if (key < N && d < RS) {
         const size_t off = row_off(b, key, N, H, h, RS) + d;
-        a.dk[off] = dka[dt][r] * a.scale;
-        a.dv[off] = dva[dt][r];
+        a.dk[off] = dka[dt][r] * unk * a.scale;
+        a.dv[off] = dva[dt][r] * unv;
       }
     }
   }
@@ -649,14 +668,15 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 
 // dQ^T of 32 queries (lane c) to its rows.
 template <int DT, int MODE>
-__device__ __forceinline__ void store_dq(const FbwdArgs& a, const f32x16 (&acc)[DT], size_t qoff,
-                                         int hf, int RS) {
+__device__ __forceinline__ void store_dq(const FbwdArgs& a, const f32x16 (&acc)[DT], float unit,
+                                         size_t qoff, int hf, int RS) {
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int qq = 0; qq < 4; ++qq) {
-      const f32x4 y = {acc[dt][4 * qq] * a.scale, acc[dt][4 * qq + 1] * a.scale,
-                       acc[dt][4 * qq + 2] * a.scale, acc[dt][4 * qq + 3] * a.scale};
+      const f32x4 y = {acc[dt][4 * qq] * unit * a.scale, acc[dt][4 * qq + 1] * unit * a.scale,
+                       acc[dt][4 * qq + 2] * unit * a.scale,
+                       acc[dt][4 * qq + 3] * unit * a.scale};
       store4m<MODE>(a.dq + qoff, dt * 32 + 8 * qq + 4 * hf, RS, y);
     }
 }
@@ -733,8 +753,10 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int d0 = 16 * kb + 8 * hf;
-    split8(load4m<MODE>(a.q + qoff, d0, RS), load4m<MODE>(a.q + qoff, d0 + 4, RS), qf[kb]);
-    split8(load4m<MODE>(a.dout + qoff, d0, RS), load4m<MODE>(a.dout + qoff, d0 + 4, RS), df[kb]);
+    split8(load4m<MODE>(a.q + qoff, d0, RS) * kScale,
+           load4m<MODE>(a.q + qoff, d0 + 4, RS) * kScale, qf[kb]);
+    split8(load4m<MODE>(a.dout + qoff, d0, RS) * kScale,
+           load4m<MODE>(a.dout + qoff, d0 + 4, RS) * kScale, df[kb]);
   }
   f32x16 acc[DT];
 #pragma unroll
@@ -742,13 +764,15 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
   const int pieces = (min(blk * kRows + kRows, N) + 31) / 32;
   const int wq_last = wq0 < N ? min(wq0 + 31, N - 1) : -1;  // -1: the wave has no query
 
-  auto to_ds = [&](const f32x16& s, f32x16& dp, int key0) {
+  // dS of a piece from S and dP, which carry 2^32 (prod) and give 2^48, or 1
+  auto to_ds = [&](const f32x16& s, f32x16& dp, int key0, float unit, float prod, float p_scale) {
+    const float sl2 = a.sl2 * unit, dlp = dl * prod, ilp = il * p_scale;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = key0 + 8 * (r / 4) + 4 * hf + (r % 4);
-      const float e = fast_exp2(fmaf(s[r], a.sl2, -m2)) * il;
+      const float e = fast_exp2(fmaf(s[r], sl2, -m2)) * ilp;
       const float p = key <= qlim ? e : 0.f;
-      dp[r] = (dp[r] - dl) * p;
+      dp[r] = (dp[r] - dlp) * p;
     }
   };
   St st[2];  // K, V
@@ -761,7 +785,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
   for (int j = 0; j < pieces; ++j) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sK : sV);
+    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sK : sV, kScale);
     __syncthreads();
     if (j + 1 < pieces) load_piece(j + 1);
     const int key0 = j * 32;
@@ -775,7 +799,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
       s = mfma_split_swapped(ka, qf[kb], s);
       dp = mfma_split_swapped(va, df[kb], dp);
     }
-    to_ds(s, dp, key0);
+    to_ds(s, dp, key0, kUnscale, kProdScale, kScale);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       bf16x8 f[3];
@@ -788,7 +812,9 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
       }
     }
   }
+  float unit = kGradUnscale;
   if (dq_bad(acc, qok, hf, RS)) {  // not all finite: the wave again with fp32 products
+    unit = 1.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
     for (int key0 = 0; key0 <= wq_last; key0 += 32) {
@@ -804,11 +830,11 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
           dp = mfma_f32(va[t], da[t], dp);
         }
       }
-      to_ds(s, dp, key0);
+      to_ds(s, dp, key0, 1.f, 1.f, 1.f);
       dq_piece_f32(acc, dp, kh, key0, N, rs, RS, c, hf);
     }
   }
-  if (qok) store_dq<DT, MODE>(a, acc, qoff, hf, RS);
+  if (qok) store_dq<DT, MODE>(a, acc, unit, qoff, hf, RS);
 }
 
 // dQ from the stored dS: per 32-key piece the lane of query c loads its dS
@@ -872,7 +898,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
     constexpr int F = decltype(fc)::value;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NV; ++i) st.store(i, sK);
+    for (int i = 0; i < NV; ++i) st.store(i, sK, kScale);
     __syncthreads();
     if (j + 1 < steps) {
 #pragma unroll
@@ -888,7 +914,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         bf16x8 f[3];
-        split8(cur[2 * kk], cur[2 * kk + 1], f);
+        split8(cur[2 * kk] * kScale, cur[2 * kk + 1] * kScale, f);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           bf16x8 kt[3];
@@ -902,7 +928,9 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
     step(std::integral_constant<int, 0>{}, j);
     if (j + 1 < steps) step(std::integral_constant<int, 1>{}, j + 1);
   }
+  float unit = kUnscale;
   if (dq_bad(acc, qok, hf, RS)) {  // not all finite: the wave again with fp32 products
+    unit = 1.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
     for (int key0 = 0; key0 <= wq_last; key0 += 32) {
@@ -914,7 +942,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
       dq_piece_f32(acc, x, kh, key0, N, rs, RS, c, hf);
     }
   }
-  if (qok) store_dq<DT, MODE>(a, acc, row_off(b, qrow, N, H, h, RS), hf, RS);
+  if (qok) store_dq<DT, MODE>(a, acc, unit, row_off(b, qrow, N, H, h, RS), hf, RS);
 }
 
 }  // namespace

@@ -22,7 +22,7 @@
 // x 32 each. K goes in steps of 32: quads of 4 consecutive k are read as fp32
 // two steps ahead, split in registers and stored as three 8-byte pieces, one
 // per plane, into the LDS stage the next step's products read (two stages, one
-// barrier a step). The splitting, 5.5 vector instructions a value, is placed
+// barrier a step). The splitting, 6.5 vector instructions a value, is placed
 // between the MFMAs, which run meanwhile. LDS planes are [rows][32] bf16 with
 // the 16-byte chunks of a row at chunk ^ (row / 4 % 4): 16 rows of one chunk,
 // the operand read, hit 16 distinct 16-byte bank groups. LayerNorm rows are
@@ -214,7 +214,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
       }
     }
     uint32_t h, m, l;
-    split2(x, y, h, m, l);
+    split2(x * kSplitScale, y * kSplitScale, h, m, l);
     ph[q] = h;
     pm[q] = m;
     pl[q] = l;
@@ -305,6 +305,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
   }
 
   bool bad = false;
+  float unscale = kSplitUnscale;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -314,6 +315,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
   if (__ballot(bad) != 0ull) {
     // an infinity among the operands (or a result that is none): the
     // wavefront's outputs again with fp32 products
+    unscale = 1.f;
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -362,7 +364,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
         if (m >= a.M) continue;
         const size_t o = a.split > 0 ? ((size_t)seg * a.M + m) * a.split + (n - seg * a.split)
                                      : (size_t)m * a.N + n;
-        float v = acc[i][j][r] + bv;
+        float v = fmaf(acc[i][j][r], unscale, bv);
         if (a.act == 1) v = gelu_tanh_g(v);
         if (a.res) v += a.res[o];
         a.y[o] = v;

@@ -2,15 +2,21 @@
 // bf16 matrix cores.
 //
 // x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 8
-// significant bits each, the differences exact. A product takes the six
+// significant bits each, the differences exact. Operands are split as 2^24 x:
+// bf16 has the exponents of fp32 but ends at 2^-133, so below 2^-111 the third
+// part of x itself, then the second, would be cut off (relative error 5e-5 at
+// 2^-120). Scaled, the parts of any fp32 value are normal bf16 values (the
+// matrix cores take subnormal ones, with fewer bits of the product). The
+// factors are powers of two, so results come out with the same bits after
+// their inverse (a product of two operands carries 2^48). A product takes the six
 // partial products of order 2^-16 and larger, hh + hm + mh + mm + hl + lh, on
 // v_mfma_f32_32x32x16_bf16 with fp32 accumulation; what is left out is below
 // 2^-25 of a product. Six of them do the work of eight v_mfma_f32_32x32x2_f32
 // in 192 matrix-core cycles instead of 512 and round the accumulator 6 times
 // per 16 k instead of 8. The parts of a value that is not finite, or that
-// rounds to infinity in bf16, hold a NaN or infinities of both signs, so its
-// products come out as NaN: kernels recompute non-finite results with fp32
-// products.
+// passes the largest finite one when scaled (from 2^104), hold a NaN or
+// infinities of both signs, so its products come out as NaN: kernels
+// recompute non-finite results with fp32 products.
 #pragma once
 
 #include "skv_common.h"
@@ -22,7 +28,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f32x16 __attribute__((ext_vector_type(16)));
 
-// Two values as three words of two parts each (the first in the low half).
+constexpr float kSplitScale = 0x1p24f;    // of every operand
+constexpr float kSplitUnscale = 0x1p-48f;  // of a product of two
+
+// Two scaled values as three words of two parts each (the first in the low half).
 // (No contraction: x is a rounded value, also where it is a product.)
 __device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
 #pragma clang fp contract(off)

@@ -105,3 +105,21 @@ def test_gemm_nonfinite_and_large(gpu_ctx, M, N):
     np.testing.assert_array_equal(got[inf], want[inf])
     fin = np.isfinite(want)
     assert (np.abs(got[fin] - want[fin]) <= tol[fin]).all()
+
+
+@pytest.mark.parametrize("M,N", [(70, 70), (1100, 1090), (4097, 4160)])
+@pytest.mark.parametrize("e", [-111, -113, -119, -126, -134, -149])
+def test_gemm_small_operands(gpu_ctx, M, N, e):
+    """Operands down to the smallest fp32 value keep every bit (three bf16 parts
+    of the value itself would lose them below 2^-111), on either side."""
+    banner(f"gemm small operands 2^{e} M={M} N={N}")
+    K = 36
+    rng = np.random.default_rng(-e)
+    with np.errstate(under="ignore"):
+        small = (rng.standard_normal((M, K)) * 2.0 ** e).astype(np.float32)
+    big = (rng.standard_normal((N, K)) * 2.0 ** 100).astype(np.float32)
+    want = small.astype(np.float64) @ big.astype(np.float64).T
+    tol = _bound(small.astype(np.float64), big.astype(np.float64), 0)
+    tol += 2.0 ** -149 - 1e-30  # (outputs as small as 2^-60: no room of _bound's own)
+    assert (np.abs(_linear(small, big) - want) <= tol).all()
+    assert (np.abs(_linear(big, small) - want.T) <= tol.T).all()
