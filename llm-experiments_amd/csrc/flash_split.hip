@@ -142,10 +142,25 @@ __device__ __forceinline__ void split_tile(const f32x16& t, int kk, bf16x8 (&f)[
          f32x4{t[8 * kk + 4], t[8 * kk + 5], t[8 * kk + 6], t[8 * kk + 7]}, f);
 }
 
+// The elements of DT tiles that are not finite, bit 16 dt + r.
+template <int DT>
+__device__ __forceinline__ uint64_t non_finite(const f32x16 (&t)[DT]) {
+  uint64_t set = 0;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) set |= (uint64_t)(finite(t[dt][r]) ? 0 : 1) << (16 * dt + r);
+  return set;
+}
+
+// Unrolling of the loops that take non-finite sums from fp32 products: they run
+// rarely and must not cost the kernels registers.
+template <int MODE>
+constexpr int kAgain = MODE == 2 ? 1 : 2;
+
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
 
 // ---------------------------------------------------------------------------
 // Forward. One workgroup per (128 queries, b, query head), rank-major: all (b,
@@ -208,9 +223,9 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
   float m_run = -INFINITY, m_true = -INFINITY, l = 0.f;
 
   // The online softmax of the piece at key0: s holds its scores in log2 units
-  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query), times unit's
-  // inverse, and gets the probabilities times p_scale.
-  auto softmax = [&](f32x16& s, int key0, float unit, float p_scale) {
+  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query) times 2^48, and
+  // gets the probabilities times 2^24.
+  auto softmax = [&](f32x16& s, int key0) {
     // A piece wholly at or below the diagonal of a wave whose 32 queries are
     // all valid masks nothing (wave-uniform test).
     float tmax = -INFINITY;
@@ -223,7 +238,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-    tmax = xor32_max(tmax) * unit;  // both halves hold the same query
+    tmax = xor32_max(tmax) * kSplitUnscale;  // both halves hold the same query
     m_true = fmaxf(m_true, tmax);
     const bool upd = tmax > m_run + 8.f;  // also true on the first piece with a key
     if (__ballot(upd) != 0ull) {          // wave-uniform branch
@@ -239,9 +254,9 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     const float m_use = m_run == -INFINITY ? 0.f : m_run;  // nothing unmasked yet
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(fmaf(s[r], unit, -m_use));
+      s[r] = fast_exp2(fmaf(s[r], kSplitUnscale, -m_use));
       l += s[r];
-      s[r] *= p_scale;
+      s[r] *= kSplitScale;
     }
   };
 
@@ -287,7 +302,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
         for (int i = 0; i < 2 * NV; ++i)
           if (i * KB / (2 * NV) == kb) stage_quad(i);
       }
-      softmax(s, key0, kSplitUnscale, kSplitScale);
+      softmax(s, key0);
       // O^T[d][query] += sum_key V[key][d] P^T[key][query]
       bf16x8 pf[2][3];
       split_tile(s, 0, pf[0]);
@@ -319,62 +334,97 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 
   // Sums that are not all finite (an infinity, a NaN or a value too large to
   // scale among the operands), or a query whose scores all came out as -inf:
-  // the wave's queries again with fp32 products, straight from global memory.
-  float unscale = kSplitUnscale;
-  bool bad = qok && !(lt > 0.f && finite(lt));
+  // taken below from fp32 products.
+  const bool row_bad = qok && !(lt > 0.f && finite(lt));
+  bool bad = row_bad;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       bad |= qok && dt * 32 + 8 * (r / 4) + 4 * hf + (r % 4) < RS && !finite(acc[dt][r]);
-  if (__ballot(bad) != 0ull) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = acl[LO ? dt : 0] = f32x16{};
-    m_run = m_true = -INFINITY;
-    l = 0.f;
-    unscale = 1.f;
-    for (int key0 = 0; key0 <= wq_last; key0 += 32) {
-      f32x16 s = f32x16{};
-      const float* kr = kh + (size_t)min(key0 + c, kv_end - 1) * rs;
-      for (int g = 0; g < D / 8; ++g) {
-        const f32x4 ka = load4m<MODE>(kr, 8 * g + 4 * hf, RS);
-        const f32x4 qa = load4m<MODE>(qp, 8 * g + 4 * hf, RS);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) s = mfma_f32(ka[t], qa[t], s);
-      }
-      s *= a.sl2;
-      softmax(s, key0, 1.f, 1.f);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const int dcol = dt * 32 + c;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = min(key0 + 8 * (r / 4) + 4 * hf + (r % 4), kv_end - 1);
-          const float vv = vh[(size_t)key * rs + (dcol < RS ? dcol : 0)];
-          acc[dt] = mfma_f32(dcol < RS ? vv : 0.f, s[r], acc[dt]);
-        }
-      }
-    }
-    lt = xor32_sum(l);
-  }
+  const bool again = __ballot(bad) != 0ull;
+  // (out may be q: the queries wait in LDS, each lane's own quads)
+  f32x4* const ql = reinterpret_cast<f32x4*>(lds) + (wave * 32 + c) * (D / 4);
+  if (again)
+    for (int g = hf; g < D / 4; g += 2) ql[g] = load4m<MODE>(qp, 4 * g, RS);
 
-  if (qi >= C) return;
   const size_t orow = ((size_t)b * C + qi) * Hq + h;
-  const float inv = qok ? 1.f / lt * unscale : 0.f;  // a valid row saw its own key: lt >= 1
+  if (qi < C) {
+    const float inv = qok ? 1.f / lt * kSplitUnscale : 0.f;  // a valid row saw its own key: lt >= 1
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
+    for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
-    for (int qq = 0; qq < 4; ++qq) {
-      const int d0 = dt * 32 + 8 * qq + 4 * hf;
-      f32x4 y = {acc[dt][4 * qq] * inv, acc[dt][4 * qq + 1] * inv, acc[dt][4 * qq + 2] * inv,
-                 acc[dt][4 * qq + 3] * inv};
-      if (!qok) y = f32x4{0.f, 0.f, 0.f, 0.f};
-      store4m<MODE>(a.out + orow * RS, d0, RS, y);
+      for (int qq = 0; qq < 4; ++qq) {
+        const int d0 = dt * 32 + 8 * qq + 4 * hf;
+        f32x4 y = {acc[dt][4 * qq] * inv, acc[dt][4 * qq + 1] * inv, acc[dt][4 * qq + 2] * inv,
+                   acc[dt][4 * qq + 3] * inv};
+        if (!qok) y = f32x4{0.f, 0.f, 0.f, 0.f};
+        store4m<MODE>(a.out + orow * RS, d0, RS, y);
+      }
+    }
+    if (hf == 0 && qok) {
+      if (a.L) a.L[orow] = lt * fast_exp2(m_run - m_true);  // relative to the true maximum
+      if (a.M) a.M[orow] = m_true * (1.f / LOG2E);          // natural units, as the scores
     }
   }
-  if (hf == 0 && qok) {
-    if (a.L) a.L[orow] = lt * fast_exp2(m_run - m_true);  // relative to the true maximum
-    if (a.M) a.M[orow] = m_true * (1.f / LOG2E);          // natural units, as the scores
+  if (!again) return;
+
+  // The elements that are not finite, and no others (a row's bits do not depend
+  // on the rows beside it), from fp32 products straight from global memory.
+  const uint64_t redo = !qok ? 0ull : row_bad ? ~0ull : non_finite(acc);
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
+  float m = -INFINITY, lsum = 0.f;
+#pragma unroll 1
+  for (int key0 = 0; key0 <= wq_last; key0 += 32) {
+    f32x16 s = f32x16{};
+    const float* kr = kh + (size_t)min(key0 + c, kv_end - 1) * rs;
+#pragma unroll kAgain<MODE>
+    for (int g = 0; g < D / 8; ++g) {
+      const f32x4 ka = load4m<MODE>(kr, 8 * g + 4 * hf, RS);
+      const f32x4 qa = ql[2 * g + hf];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s = mfma_f32(ka[t], qa[t], s);
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = key0 + 8 * (r / 4) + 4 * hf + (r % 4) <= qlim ? s[r] * a.sl2 : -INFINITY;
+      tmax = fmaxf(tmax, s[r]);
+    }
+    const float mn = fmaxf(m, xor32_max(tmax)), m_use = mn == -INFINITY ? 0.f : mn;
+    const float alpha = fast_exp2(m - m_use);  // m = -inf: 0
+    m = mn;
+    lsum *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = fast_exp2(s[r] - m_use);
+      lsum += s[r];
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const int d = dt * 32 + c;
+      o[dt] *= alpha;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = min(key0 + 8 * (r / 4) + 4 * hf + (r % 4), kv_end - 1);
+        const float vv = vh[(size_t)key * rs + (d < RS ? d : 0)];
+        o[dt] = mfma_f32(d < RS ? vv : 0.f, s[r], o[dt]);
+      }
+    }
+  }
+  lsum = xor32_sum(lsum);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int d = dt * 32 + 8 * (r / 4) + 4 * hf + (r % 4);
+      if (d < RS && ((redo >> (16 * dt + r)) & 1) != 0) a.out[orow * RS + d] = o[dt][r] / lsum;
+    }
+  if (row_bad && hf == 0) {
+    if (a.L) a.L[orow] = lsum;
+    if (a.M) a.M[orow] = m * (1.f / LOG2E);
   }
 }
 
@@ -478,7 +528,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   // the query block adds a whole row of tiles): key c, rows 4 hf + ...
   float* dsw = nullptr;
   if constexpr (DSO) dsw = ds_tile(a, bh, 0, wk0 >> 5) + ds_key_pos(c) + 128 * hf;
-  auto store_ds = [&](auto interior, const f32x16& ds, float unit, int q0) {
+  auto store_ds = [&](auto interior, const f32x16& ds, int q0) {
     // for each slot the 32 lanes of a half write one query's 128-byte tile
     // row, past the caches (read once, later)
     if (decltype(interior)::value || krow < N) {
@@ -486,7 +536,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (decltype(interior)::value || q0 + 8 * (r / 4) + 4 * hf + (r % 4) < N)
-          __builtin_nontemporal_store(ds[r] * unit, tp + (8 * (r / 4) + (r % 4)) * 32);
+          __builtin_nontemporal_store(ds[r] * kDsUnscale, tp + (8 * (r / 4) + (r % 4)) * 32);
     }
   };
 
@@ -569,7 +619,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
             else split_tile(dp, i - 2, df[i - 2]);
           }
       }
-    if constexpr (DSO) store_ds(interior, dp, kDsUnscale, q0);
+    if constexpr (DSO) store_ds(interior, dp, q0);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -600,23 +650,34 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
     else piece(std::false_type{}, q0);
   }
 
-  // Sums that are not all finite: the wave's keys again with fp32 products,
-  // straight from global memory.
-  float unv = kUnscale, unk = kGradUnscale;
+  // dva[dt][r], dka[dt][r]: key wk0 + 8(r/4) + 4hf + r%4, d = dt*32 + c
   bool bad = false;
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DT; ++dt) {
+    const int d = dt * 32 + c;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      bad |= wk0 + 8 * (r / 4) + 4 * hf + (r % 4) < N && dt * 32 + c < RS &&
-             !(finite(dva[dt][r]) && finite(dka[dt][r]));
+    for (int r = 0; r < 16; ++r) {
+      const int key = wk0 + 8 * (r / 4) + 4 * hf + (r % 4);
+      if (key < N && d < RS) {
+        const size_t off = row_off(b, key, N, H, h, RS) + d;
+        a.dk[off] = dka[dt][r] * kGradUnscale * a.scale;
+        a.dv[off] = dva[dt][r] * kUnscale;
+        bad |= !(finite(dva[dt][r]) && finite(dka[dt][r]));
+      }
+    }
+  }
+  // Sums that are not all finite: those elements of the wave's keys (and of
+  // dS), and no others, from fp32 products, straight from global memory.
   if (__ballot(bad) != 0ull) {
+    const uint64_t redo_v = non_finite(dva), redo_k = non_finite(dka);
+    f32x16 ev[DT], ek[DT];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) dva[dt] = dka[dt] = f32x16{};
-    unv = unk = 1.f;
+    for (int dt = 0; dt < DT; ++dt) ev[dt] = ek[dt] = f32x16{};
+#pragma unroll 1
     for (int q0 = wk0; q0 < N; q0 += 32) {
       f32x16 s = f32x16{}, dp = f32x16{};
       const size_t qo = (size_t)min(q0 + c, N - 1) * rs;
+#pragma unroll kAgain<MODE>
       for (int g = 0; g < D / 8; ++g) {
         const int d0 = 8 * g + 4 * hf;
         const f32x4 qa = load4m<MODE>(qh + qo, d0, RS), da = load4m<MODE>(dh + qo, d0, RS);
@@ -635,32 +696,41 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
         s[r] = (krow <= query && query < N) ? e : 0.f;
         dp[r] = s[r] * (dp[r] - a.delta[sr]);
       }
-      if constexpr (DSO) store_ds(std::false_type{}, dp, 1.f, q0);
+      if (DSO && krow < N) {  // dS where it is not finite
+        float* tp = dsw + (size_t)(q0 >> 5) * ((N + 31) >> 5) * 1024;
+        uint32_t bad_ds = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)  // (a query past N: this tile's own memory, not used)
+          bad_ds |= (uint32_t)(finite(tp[(8 * (r / 4) + (r % 4)) * 32]) ? 0 : 1) << r;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (((bad_ds >> r) & 1) != 0 && q0 + 8 * (r / 4) + 4 * hf + (r % 4) < N)
+            tp[(8 * (r / 4) + (r % 4)) * 32] = dp[r];
+      }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const int dcol = dt * 32 + c;
+        const int d = dt * 32 + c;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const size_t o = (size_t)min(q0 + 8 * (r / 4) + 4 * hf + (r % 4), N - 1) * rs +
-                           (dcol < RS ? dcol : 0);
+                           (d < RS ? d : 0);
           const float xo = dh[o], xq = qh[o];
-          dva[dt] = mfma_f32(s[r], dcol < RS ? xo : 0.f, dva[dt]);
-          dka[dt] = mfma_f32(dp[r], dcol < RS ? xq : 0.f, dka[dt]);
+          ev[dt] = mfma_f32(s[r], d < RS ? xo : 0.f, ev[dt]);
+          ek[dt] = mfma_f32(dp[r], d < RS ? xq : 0.f, ek[dt]);
         }
       }
     }
-  }
-  // dva[dt][r], dka[dt][r]: key wk0 + 8(r/4) + 4hf + r%4, d = dt*32 + c
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    const int d = dt * 32 + c;
+    for (int dt = 0; dt < DT; ++dt) {
+      const int d = dt * 32 + c;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = wk0 + 8 * (r / 4) + 4 * hf + (r % 4);
-      if (key < N && d < RS) {
-        const size_t off = row_off(b, key, N, H, h, RS) + d;
-        a.dk[off] = dka[dt][r] * unk * a.scale;
-        a.dv[off] = dva[dt][r] * unv;
+      for (int r = 0; r < 16; ++r) {
+        const int key = wk0 + 8 * (r / 4) + 4 * hf + (r % 4);
+        if (key < N && d < RS) {
+          const size_t off = row_off(b, key, N, H, h, RS) + d;
+          if ((redo_k >> (16 * dt + r)) & 1) a.dk[off] = ek[dt][r] * a.scale;
+          if ((redo_v >> (16 * dt + r)) & 1) a.dv[off] = ev[dt][r];
+        }
       }
     }
   }
@@ -681,31 +751,45 @@ __device__ __forceinline__ void store_dq(const FbwdArgs& a, const f32x16 (&acc)[
     }
 }
 
-// acc[dt] += K^T[d][key] ds[key][query] with fp32 products, keys key0 .. + 31
-// straight from global memory.
-template <int DT>
-__device__ __forceinline__ void dq_piece_f32(f32x16 (&acc)[DT], const f32x16& ds, const float* kh,
-                                             int key0, int N, uint32_t rs, int RS, int c, int hf) {
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    const int dcol = dt * 32 + c;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = min(key0 + 8 * (r / 4) + 4 * hf + (r % 4), N - 1);
-      const float kv = kh[(size_t)key * rs + (dcol < RS ? dcol : 0)];
-      acc[dt] = mfma_f32(dcol < RS ? kv : 0.f, ds[r], acc[dt]);
-    }
-  }
-}
-template <int DT>
-__device__ __forceinline__ bool dq_bad(const f32x16 (&acc)[DT], bool qok, int hf, int RS) {
+// dQ of a wave's queries, and where it is not finite, those elements and no
+// others from fp32 products: form(key0) gives dS of the piece at key0.
+template <int DT, int MODE, typename F>
+__device__ __forceinline__ void finish_dq(const FbwdArgs& a, const f32x16 (&acc)[DT], float unit,
+                                          size_t qoff, bool qok, int wq_last, const float* kh,
+                                          uint32_t rs, int RS, int c, int hf, F form) {
   bool bad = false;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       bad |= qok && dt * 32 + 8 * (r / 4) + 4 * hf + (r % 4) < RS && !finite(acc[dt][r]);
-  return __ballot(bad) != 0ull;
+  if (qok) store_dq<DT, MODE>(a, acc, unit, qoff, hf, RS);
+  if (__ballot(bad) == 0ull) return;
+  const uint64_t redo = qok ? non_finite(acc) : 0ull;
+  f32x16 e[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) e[dt] = f32x16{};
+#pragma unroll 1
+  for (int key0 = 0; key0 <= wq_last; key0 += 32) {
+    const f32x16 ds = form(key0);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const int d = dt * 32 + c;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = min(key0 + 8 * (r / 4) + 4 * hf + (r % 4), a.N - 1);
+        const float kv = kh[(size_t)key * rs + (d < RS ? d : 0)];
+        e[dt] = mfma_f32(d < RS ? kv : 0.f, ds[r], e[dt]);
+      }
+    }
+  }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int d = dt * 32 + 8 * (r / 4) + 4 * hf + (r % 4);
+      if (d < RS && ((redo >> (16 * dt + r)) & 1) != 0) a.dq[qoff + d] = e[dt][r] * a.scale;
+    }
 }
 
 // dQ and the row deltas; rank 0 = the last query block (the most keys).
@@ -812,29 +896,23 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
       }
     }
   }
-  float unit = kGradUnscale;
-  if (dq_bad(acc, qok, hf, RS)) {  // not all finite: the wave again with fp32 products
-    unit = 1.f;
+  finish_dq<DT, MODE>(a, acc, kGradUnscale, qoff, qok, wq_last, kh, rs, RS, c, hf, [&](int key0) {
+    f32x16 s = f32x16{}, dp = f32x16{};
+    const size_t ko = (size_t)min(key0 + c, N - 1) * rs;
+#pragma unroll kAgain<MODE>
+    for (int g = 0; g < D / 8; ++g) {
+      const int d0 = 8 * g + 4 * hf;
+      const f32x4 ka = load4m<MODE>(kh + ko, d0, RS), va = load4m<MODE>(vh + ko, d0, RS);
+      const f32x4 qa = load4m<MODE>(a.q + qoff, d0, RS), da = load4m<MODE>(a.dout + qoff, d0, RS);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
-    for (int key0 = 0; key0 <= wq_last; key0 += 32) {
-      f32x16 s = f32x16{}, dp = f32x16{};
-      const size_t ko = (size_t)min(key0 + c, N - 1) * rs;
-      for (int g = 0; g < D / 8; ++g) {
-        const int d0 = 8 * g + 4 * hf;
-        const f32x4 ka = load4m<MODE>(kh + ko, d0, RS), va = load4m<MODE>(vh + ko, d0, RS);
-        const f32x4 qa = load4m<MODE>(a.q + qoff, d0, RS), da = load4m<MODE>(a.dout + qoff, d0, RS);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          s = mfma_f32(ka[t], qa[t], s);
-          dp = mfma_f32(va[t], da[t], dp);
-        }
+      for (int t = 0; t < 4; ++t) {
+        s = mfma_f32(ka[t], qa[t], s);
+        dp = mfma_f32(va[t], da[t], dp);
       }
-      to_ds(s, dp, key0, 1.f, 1.f, 1.f);
-      dq_piece_f32(acc, dp, kh, key0, N, rs, RS, c, hf);
     }
-  }
-  if (qok) store_dq<DT, MODE>(a, acc, unit, qoff, hf, RS);
+    to_ds(s, dp, key0, 1.f, 1.f, 1.f);
+    return dp;
+  });
 }
 
 // dQ from the stored dS: per 32-key piece the lane of query c loads its dS
@@ -928,21 +1006,16 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
     step(std::integral_constant<int, 0>{}, j);
     if (j + 1 < steps) step(std::integral_constant<int, 1>{}, j + 1);
   }
-  float unit = kUnscale;
-  if (dq_bad(acc, qok, hf, RS)) {  // not all finite: the wave again with fp32 products
-    unit = 1.f;
+  finish_dq<DT, MODE>(a, acc, kUnscale, row_off(b, qrow, N, H, h, RS), qok, wq_last, kh, rs, RS, c,
+                      hf, [&](int key0) {
+    f32x4 x[4];
+    load_ds(key0, x);
+    mask_ds(key0, x);
+    f32x16 y;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
-    for (int key0 = 0; key0 <= wq_last; key0 += 32) {
-      load_ds(key0, ds[0][0]);
-      mask_ds(key0, ds[0][0]);
-      f32x16 x;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) x[r] = ds[0][0][r >> 2][r & 3];
-      dq_piece_f32(acc, x, kh, key0, N, rs, RS, c, hf);
-    }
-  }
-  if (qok) store_dq<DT, MODE>(a, acc, unit, row_off(b, qrow, N, H, h, RS), hf, RS);
+    for (int r = 0; r < 16; ++r) y[r] = x[r >> 2][r & 3];
+    return y;
+  });
 }
 
 }  // namespace

@@ -14,9 +14,9 @@
 // 2048 x 3072 x 768 with LayerNorm 137 -> 67 us, 2048 x 768 x 3072 220 -> 79
 // us, 111 x 640 x 2560 192 -> 48 us; error against float64 (relative
 // 2-norm) 5.0e-7 -> 4.2e-7 at K = 768 and 9.9e-7 -> 8.6e-7 at K = 3072.
-// A wavefront whose sums are not all finite (an infinity, or a value that
-// rounds to one in bf16, among the operands) computes them again on
-// v_mfma_f32_32x32x2_f32, which gives what fp32 products give.
+// Outputs that are not finite (an infinity, or a value too large to split,
+// among the operands) are computed again on v_mfma_f32_32x32x2_f32, which
+// gives what fp32 products give.
 //
 // Design: a workgroup computes BM x BN outputs, its wavefronts 64 x 64 or 32
 // x 32 each. K goes in steps of 32: quads of 4 consecutive k are read as fp32
@@ -304,71 +304,79 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
     step(std::integral_constant<int, 1>{}, s + 1);
   }
 
+  // Output tile (i, j) of the wavefront with fp32 products, straight from
+  // global memory: k 8 g + 4 hf + t in step (g, t).
+  auto tile_f32 = [&](int i, int j) {
+    const float* xr = a.x + (size_t)min(m0 + wm * WM + i * 32 + c, a.M - 1) * a.K;
+    const float* wr = a.wt + (size_t)min(n0 + wn * WN + j * 32 + c, a.N - 1) * a.K;
+    float mi = 0.f, ri = 0.f;
+    if constexpr (LN) {  // one row per lane here, as row_stats
+      float sm = 0.f, sq = 0.f;
+      for (int k = 0; k < a.K; ++k) {
+        const float v = xr[k] - xr[0];
+        sm += v;
+        sq += v * v;
+      }
+      const float ms = sm / a.K;
+      mi = xr[0] + ms;
+      ri = 1.f / sqrtf(fmaxf(sq / a.K - ms * ms, 0.f) + a.ln_eps);
+    }
+    f32x16 e = f32x16{};
+    for (int k0 = 0; k0 < a.K; k0 += 8) {
+      const bool in = k0 + 4 * hf < a.K;  // (K % 4 == 0)
+      const int k = in ? k0 + 4 * hf : 0;
+      f32x4 x = *reinterpret_cast<const f32x4*>(xr + k);
+      f32x4 w = *reinterpret_cast<const f32x4*>(wr + k);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (LN) x[t] = (x[t] - mi) * ri * a.ln_g[k + t] + a.ln_b[k + t];
+        e = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x[t] : 0.f, in ? w[t] : 0.f, e, 0, 0, 0);
+      }
+    }
+    return e;
+  };
+  // Outputs that are not finite (an infinity among the operands, a value too
+  // large to scale, or a result that is none) take the value of the fp32
+  // products; the others keep theirs, so a row's bits do not depend on the rows
+  // and columns beside it.
   bool bad = false;
-  float unscale = kSplitUnscale;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
-  if (__ballot(bad) != 0ull) {
-    // an infinity among the operands (or a result that is none): the
-    // wavefront's outputs again with fp32 products
-    unscale = 1.f;
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) acc[i][j] = f32x16{};
-#pragma unroll
-    for (int i = 0; i < TI; ++i) {
-      const int m = min(m0 + wm * WM + i * 32 + c, a.M - 1);
-      const float* xr = a.x + (size_t)m * a.K;
-      float mi = 0.f, ri = 0.f;
-      if constexpr (LN) {  // one row per lane here, as row_stats
-        float sm = 0.f, sq = 0.f;
-        for (int k = 0; k < a.K; ++k) {
-          const float v = xr[k] - xr[0];
-          sm += v;
-          sq += v * v;
-        }
-        const float ms = sm / a.K;
-        mi = xr[0] + ms;
-        ri = 1.f / sqrtf(fmaxf(sq / a.K - ms * ms, 0.f) + a.ln_eps);
-      }
-      for (int k = hf; k < a.K; k += 2) {
-        float x = xr[k];
-        if constexpr (LN) x = (x - mi) * ri * a.ln_g[k] + a.ln_b[k];
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-          const int n = min(n0 + wn * WN + j * 32 + c, a.N - 1);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, a.wt[(size_t)n * a.K + k],
-                                                           acc[i][j], 0, 0, 0);
-        }
-      }
-    }
-  }
+      for (int r = 0; r < 16; ++r) bad |= !finite(acc[i][j][r]);
+  const bool redo = __ballot(bad) != 0ull;
 
   // acc[i][j][r]: row m0 + WM wm + 32 i + 8 (r/4) + 4 hf + r%4, column n0 + WN wn + 32 j + c
 #pragma unroll
   for (int j = 0; j < TJ; ++j) {
     const int n = n0 + wn * WN + j * 32 + c;
-    if (n >= a.N) continue;
-    const float bv = a.bias ? a.bias[n] : 0.f;
+    const float bv = a.bias && n < a.N ? a.bias[n] : 0.f;
     const int seg = a.split > 0 ? n / a.split : 0;
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int i = 0; i < TI; ++i) {
+      f32x16 y;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) y[r] = fmaf(acc[i][j][r], kSplitUnscale, bv);
+      if (redo) {
+        const f32x16 e = tile_f32(i, j);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] = finite(acc[i][j][r]) ? y[r] : e[r] + bv;
+      }
+      if (n >= a.N) continue;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
         if (m >= a.M) continue;
         const size_t o = a.split > 0 ? ((size_t)seg * a.M + m) * a.split + (n - seg * a.split)
                                      : (size_t)m * a.N + n;
-        float v = fmaf(acc[i][j][r], unscale, bv);
+        float v = y[r];
         if (a.act == 1) v = gelu_tanh_g(v);
         if (a.res) v += a.res[o];
         a.y[o] = v;
       }
+    }
   }
 }
 

@@ -15,8 +15,8 @@
 // in 192 matrix-core cycles instead of 512 and round the accumulator 6 times
 // per 16 k instead of 8. The parts of a value that is not finite, or that
 // passes the largest finite one when scaled (from 2^104), hold a NaN or
-// infinities of both signs, so its products come out as NaN: kernels
-// recompute non-finite results with fp32 products.
+// infinities of both signs, so its products come out as NaN: kernels take
+// those results, and no others, from fp32 products.
 #pragma once
 
 #include "skv_common.h"
@@ -27,6 +27,8 @@ typedef float split_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
 
 constexpr float kSplitScale = 0x1p24f;    // of every operand
 constexpr float kSplitUnscale = 0x1p-48f;  // of a product of two

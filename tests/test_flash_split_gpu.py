@@ -21,6 +21,15 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
 
 
+def flash_fwd_into(out, q, k, v, N, H, D):
+    from simple_llm_amd import _lib
+    st = torch.empty(2 * N * H, device=q.device)
+    _lib.check(_lib.lib().skv_flash_fwd(out.data_ptr(), st.data_ptr(), st[N * H:].data_ptr(),
+                                        q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, N, H, D,
+                                        float(1 / np.sqrt(D)), _lib.stream_handle(q.device)),
+               "skv_flash_fwd")
+
+
 def _dev(x):
     return torch.from_numpy(np.ascontiguousarray(x, np.float32)).cuda()
 
@@ -128,3 +137,36 @@ def test_small_operands(gpu_ctx, D, scale, fast):
     s = np.einsum("qhd,khd->hqk", t["q"].astype(np.float64), t["k"].astype(np.float64))
     s = np.where(np.tril(np.ones((N, N), bool)), s / np.sqrt(D), -np.inf).max(-1).T
     assert _rel(M.cpu().numpy().reshape(N, H).astype(np.float64), s) < 5e-6
+
+
+@pytest.mark.parametrize("D", [20, 50, 64, 96, 128])
+@pytest.mark.parametrize("what", ["q", "k", "v", "go"])
+def test_rows_beside_non_finite_ones_keep_their_bits(gpu_ctx, D, what):
+    """An infinite element at row 40 leaves the bits of every row that does not
+    see it: queries before it (queries other than 40 where it is a query's),
+    keys after it, and the other head. (Rows 32 to 63 share a piece with it, where
+    a masked pair weighs 0 times infinity.)"""
+    banner(f"flash rows beside a non-finite {what} D={D}")
+    N, H, at = 150, 2, 40
+    rng = np.random.default_rng(D)
+    t = {n: rng.standard_normal((N, H, D)).astype(np.float32) for n in ("q", "k", "v", "go")}
+    runs = []
+    for bad in (False, True):
+        if bad:
+            t[what][at, 0, 5] = np.inf
+        f = {n: _dev(x.reshape(N, H * D)) for n, x in t.items()}
+        o, L, M = flash_fwd(f["q"], f["k"], f["v"], 1, N, H, D)
+        row = f["q"].clone()  # the output in place of the queries
+        flash_fwd_into(row, row, f["k"], f["v"], N, H, D)
+        assert torch.equal(row.view(torch.int32), o.view(torch.int32))
+        for fast in (False, True):
+            grads = flash_bwd(f["q"], f["k"], f["v"], o, L, M, f["go"], 1, N, H, D, fast=fast)
+            runs.append([x.cpu().numpy().reshape(N, H, -1) for x in (o, L, M, *grads)])
+    own = what in ("q", "go")  # a query's operand
+    queries = np.delete(np.arange(N), at) if own else np.arange(32)
+    keys = np.arange(64, N) if own else np.arange(0)  # (queries from 40 on see every key)
+    for a, b in zip(runs[:2], runs[2:]):
+        for i, rows in enumerate((queries,) * 4 + (keys,) * 2):
+            np.testing.assert_array_equal(a[i][rows, 0], b[i][rows, 0])
+            np.testing.assert_array_equal(a[i][:, 1], b[i][:, 1])
+    assert what == "go" or not np.isfinite(runs[2][0][at:, 0]).all()

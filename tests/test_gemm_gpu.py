@@ -123,3 +123,25 @@ def test_gemm_small_operands(gpu_ctx, M, N, e):
     tol += 2.0 ** -149 - 1e-30  # (outputs as small as 2^-60: no room of _bound's own)
     assert (np.abs(_linear(small, big) - want) <= tol).all()
     assert (np.abs(_linear(big, small) - want.T) <= tol.T).all()
+
+
+@pytest.mark.parametrize("ln", [False, True])
+@pytest.mark.parametrize("M,N", [(70, 70), (1100, 1090), (4097, 4160)])
+def test_gemm_rows_beside_non_finite_ones_keep_their_bits(gpu_ctx, M, N, ln):
+    """An infinite or NaN operand changes its own row (or column) alone."""
+    banner(f"gemm rows beside non-finite ones M={M} N={N} ln={ln}")
+    K = 44
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    g = (rng.standard_normal(K).astype(np.float32), rng.standard_normal(K).astype(np.float32))
+    for ws in (True, False) if ln else (False,):
+        clean = _linear(x, w, ln=g if ln else None, ws=ws)
+        xb, wb = x.copy(), w.copy()
+        xb[[2, 40], 5] = np.inf, np.nan
+        wb[[1, N - 1], 7] = -np.inf, np.float32(3e38)
+        got = _linear(xb, wb, ln=g if ln else None, ws=ws)
+        rows, cols = np.ones(M, bool), np.ones(N, bool)
+        rows[[2, 40]] = cols[[1, N - 1]] = False
+        np.testing.assert_array_equal(got[np.ix_(rows, cols)], clean[np.ix_(rows, cols)])
+        assert not np.isfinite(got[~rows]).any() and np.isinf(got[rows][:, 1]).all()
