@@ -131,8 +131,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_of(const float* p, long fl
 
 // One workgroup: BM x BN outputs, (BM / WM) * (BN / WN) wavefronts of WM x
 // WN. LN: LayerNorm of the x values as they are split (calls without the
-// workspace for k_layernorm_rows).
-template <int BM, int BN, int WM, int WN, bool LN>
+// workspace for k_layernorm_rows). LONG: rows too long for 32-bit offsets into a
+// tile, read through 64-bit addresses.
+template <int BM, int BN, int WM, int WN, bool LN, bool LONG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a) {
   constexpr int NT = (BM / WM) * (BN / WN) * 64;
   constexpr int TI = WM / 32, TJ = WN / 32;          // 32 x 32 tiles of a wavefront
@@ -190,6 +191,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
   } set[2];
   auto load_quad = [&](Set& r, int k0, int u) {  // quad u: of x, then of w
     const int kk = k0 + kq;
+    if constexpr (LONG) {
+      const int row = u < QA ? m0 + ((tid + NT * u) >> 3) : n0 + ((tid + NT * (u - QA)) >> 3);
+      const bool in = kk < a.K && row < (u < QA ? a.M : a.N);
+      const float* p = (u < QA ? a.x : a.wt) + (in ? (size_t)row * a.K + kk : 0);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p);
+      r.q[u] = in ? v : f32x4{0.f, 0.f, 0.f, 0.f};
+      return;
+    }
     const uint32_t past = kk < a.K ? 0u : 0xffffffffu;
     r.q[u] = u < QA ? buf_load(bx, (offx[u < QA ? u : 0] + kk * 4u) | past)
                     : buf_load(bw, (offw[u < QA ? 0 : u - QA] + kk * 4u) | past);
@@ -380,12 +389,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void k_gemm(GemmArgs a)
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool LN = false>
+template <int BM, int BN, int WM, int WN, bool LN = false, bool LONG = false>
 int launch_gemm(GemmArgs a, hipStream_t s) {
   a.mt = (a.M + BM - 1) / BM;
   const long nt = ((a.N + BN - 1) / BN + kXCD - 1) / kXCD * kXCD;
   SKV_REQUIRE(nt * a.mt < (1L << 31), SKV_E_UNSUPPORTED, "skv_linear: M=%d too large", a.M);
-  hipLaunchKernelGGL((k_gemm<BM, BN, WM, WN, LN>), dim3((unsigned)(nt * a.mt)),
+  hipLaunchKernelGGL((k_gemm<BM, BN, WM, WN, LN, LONG>), dim3((unsigned)(nt * a.mt)),
                      dim3((BM / WM) * (BN / WN) * 64), 0, s, a);
   return check_launch("skv_linear");
 }
@@ -401,10 +410,11 @@ int gemm_linear(float* y, const float* x, const float* w_t, const float* bias,
                 hipStream_t s) {
   GemmArgs a{y, x, w_t, bias, residual, ln_gamma, ln_beta, ln_eps, M, N, K, activation,
              split_cols, 0};
-  SKV_REQUIRE((long)256 * K * 4 < (1L << 32), SKV_E_UNSUPPORTED,
-              "skv_linear: K=%d too large for a tile's buffer", K);
+  const bool lng = (long)256 * K * 4 >= (1L << 32);  // 256 rows past a buffer's 32-bit range
   if (ln_gamma != nullptr) {
-    if (norm == nullptr) return launch_gemm<64, 64, 32, 32, true>(a, s);
+    if (norm == nullptr)
+      return lng ? launch_gemm<64, 64, 32, 32, true, true>(a, s)
+                 : launch_gemm<64, 64, 32, 32, true>(a, s);
     hipLaunchKernelGGL(k_layernorm_rows, dim3((M + 3) / 4), dim3(256), 0, s, norm, x, ln_gamma,
                        ln_beta, M, K, ln_eps);
     const int rc = check_launch("skv_linear");
@@ -412,6 +422,7 @@ int gemm_linear(float* y, const float* x, const float* w_t, const float* bias,
     a.x = norm;
     a.ln_g = a.ln_b = nullptr;
   }
+  if (lng) return launch_gemm<64, 64, 32, 32, false, true>(a, s);
   // Tiles by how they fill the chip's 256 CUs (measured on MI355X, us):
   //  - 256 x 128 where there are more than two rounds of them: the fewest
   //    values split per product (2048 x 50304 x 768: 853, 128 x 64 955, 64 x

@@ -145,3 +145,35 @@ def test_gemm_rows_beside_non_finite_ones_keep_their_bits(gpu_ctx, M, N, ln):
         rows[[2, 40]] = cols[[1, N - 1]] = False
         np.testing.assert_array_equal(got[np.ix_(rows, cols)], clean[np.ix_(rows, cols)])
         assert not np.isfinite(got[~rows]).any() and np.isinf(got[rows][:, 1]).all()
+
+
+@pytest.mark.parametrize("K", [(1 << 22) - 4, 1 << 22, (1 << 22) + 36])
+def test_gemm_long_rows(gpu_ctx, K):
+    """Rows on both sides of a tile's 32-bit byte range. Values of -1, 0 and 1:
+    every sum is exact. With LayerNorm: 1e-3, above a random walk of the 1.6 M
+    roundings of a sum (4e-5)."""
+    banner(f"gemm long rows K={K}")
+    from simple_llm_amd import _lib
+    L = _lib.lib()
+    M, N = 67, 5
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randint(-1, 2, (M, K), device="cuda", generator=gen).float()
+    w = torch.randint(-1, 2, (N, K), device="cuda", generator=gen).float()
+    g = torch.rand(K, device="cuda", generator=gen) + 0.5
+    b = torch.rand(K, device="cuda", generator=gen)
+    x64 = x.double()
+    norm = (x64 - x64.mean(1, keepdim=True)) / torch.sqrt(x64.var(1, unbiased=False, keepdim=True)
+                                                         + 1e-5) * g + b
+    ws = torch.zeros(L.skv_linear_workspace_bytes(M, N, K), dtype=torch.uint8, device="cuda")
+    for ln, buf in ((False, None), (True, None), (True, ws)):
+        y = torch.full((M, N), float("nan"), device="cuda")
+        _lib.check(L.skv_linear(y.data_ptr(), x.data_ptr(), w.data_ptr(), None, None,
+                                g.data_ptr() if ln else None, b.data_ptr() if ln else None, 1e-5,
+                                M, N, K, 0, 0, buf.data_ptr() if buf is not None else None,
+                                buf.numel() if buf is not None else 0, _lib.stream_handle()),
+                   "skv_linear")
+        want = (norm if ln else x64) @ w.double().T.contiguous()
+        if ln:
+            assert float((y - want).norm() / want.norm()) < 1e-3
+        else:
+            assert torch.equal(y.double(), want)
