@@ -94,15 +94,24 @@ def kv_cache_create(ctx: GPUContext, config: KVCacheConfig) -> KVCache:
     else:
         rows = B * config.max_seq_len
 
+    # A layer's fills, and after them (16-byte aligned, zero-filled together) the
+    # workspace of its one-launch decode steps where the sizes can take those.
+    step = 0
+    if (config.block_size <= 0 and _step_sizes(B, config.n_heads, n_kv, config.head_dim)
+            and ctx.device.type == "cuda"):
+        step = int(_lib.lib().skv_decode_direct_workspace_bytes(B, config.n_heads,
+                                                                config.head_dim, _STEP_SPLIT))
+    at = -(-B // 4) * 4
     layers: List[KVCacheLayer] = []
     for _ in range(config.n_layers):
         k = torch.zeros((rows, e_kv), dtype=config.dtype, device=ctx.device)
         v = torch.zeros((rows, e_kv), dtype=config.dtype, device=ctx.device)
+        state = torch.zeros(at + -(-step // 4), dtype=torch.int32, device=ctx.device)
         layers.append(KVCacheLayer(
             k_cache=GPUBuffer2D(buffer=k, shape=(rows, e_kv), size=rows * e_kv),
             v_cache=GPUBuffer2D(buffer=v, shape=(rows, e_kv), size=rows * e_kv),
-            lens=torch.zeros(B, dtype=torch.int32, device=ctx.device),
-            host_lens=np.zeros(B, dtype=np.int64)))
+            lens=state[:B], host_lens=np.zeros(B, dtype=np.int64),
+            step_ws=state[at:] if step else None))
 
     return KVCache(layers=layers, batch_size=B, max_seq_len=config.max_seq_len, current_len=0,
                    n_heads=config.n_heads, head_dim=config.head_dim, n_kv_heads=n_kv,
@@ -263,22 +272,15 @@ def _workspace(ctx: GPUContext, nbytes: int) -> torch.Tensor:
 _STEP_PAIRS = 256
 _STEP_BYTES = 1 << 20
 _STEP_SPLIT = 4
-_STEP_STREAMS = 16
 
 
-def _step_workspace(ctx: GPUContext, stream: int):
-    """The one-launch step's workspace (zero-filled once; its counters are zero
-    between calls) for this stream, of one size for every shape that takes
-    it, or None: under a capture that would own the allocation, or past the
-    streams a context keeps one for."""
-    ws = ctx.step_workspaces.get(stream)
-    if ws is None:
-        if len(ctx.step_workspaces) >= _STEP_STREAMS or torch.cuda.is_current_stream_capturing():
-            return None
-        need = _lib.lib().skv_decode_direct_workspace_bytes(1, _STEP_PAIRS, 128, _STEP_SPLIT)
-        ws = ctx.step_workspaces.setdefault(
-            stream, torch.zeros(need, dtype=torch.uint8, device=ctx.device))
-    return ws
+def _step_sizes(B: int, n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
+    """Whether a contiguous cache of these sizes can take one-launch decode steps.
+    Its layers then hold the step's workspace (arrival counters, zero between
+    calls, and partials): with the fills, which already make calls on one layer
+    stream ordered, so the route of a call does not depend on its stream, and a
+    captured call has the bits of an eager one."""
+    return n_heads == n_kv_heads and head_dim in (64, 128) and B * n_heads < _STEP_PAIRS
 
 
 _WS_BYTES: dict = {}
@@ -460,20 +462,18 @@ def kv_cache_append_attend(ctx: GPUContext, cache: KVCache, layer_idx: int, new_
     D, sc = cache.head_dim, float(scale) if scale is not None else 1.0 / math.sqrt(cache.head_dim)
     stream = _lib.stream_handle(dev)
     kc, vc = layer.k_cache.buffer.data_ptr(), layer.v_cache.buffer.data_ptr()
-    if (not cache.paged and cache.n_heads == cache.n_kv_heads and D in (64, 128)
-            and cache.batch_size * cache.n_heads < _STEP_PAIRS and not (kc | vc) & 15
+    ws = layer.step_ws
+    if (ws is not None and not (kc | vc) & 15
             and 2 * max_len * D * layer.k_cache.buffer.element_size() <= _STEP_BYTES):
-        ws = _step_workspace(ctx, stream)
-        if ws is not None:
-            rc = L.skv_append_decode_attn_step(
-                out.data_ptr(), q.data_ptr(), kc, vc, new_k.data_ptr(), new_v.data_ptr(),
-                layer.lens.data_ptr(), cache.batch_size, cache.n_heads, D, cache.max_seq_len, sc,
-                _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype),
-                _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype), _STEP_SPLIT, ws.data_ptr(),
-                ws.numel(), stream)
-            _lib.check(rc, "skv_append_decode_attn_step")
-            layer.host_lens = after
-            return after.copy()
+        rc = L.skv_append_decode_attn_step(
+            out.data_ptr(), q.data_ptr(), kc, vc, new_k.data_ptr(), new_v.data_ptr(),
+            layer.lens.data_ptr(), cache.batch_size, cache.n_heads, D, cache.max_seq_len, sc,
+            _lib.dtype_code(cache.dtype), _lib.dtype_code(new_k.dtype),
+            _lib.dtype_code(q.dtype), _lib.dtype_code(out.dtype), _STEP_SPLIT, ws.data_ptr(),
+            ws.numel() * 4, stream)
+        _lib.check(rc, "skv_append_decode_attn_step")
+        layer.host_lens = after
+        return after.copy()
     # every fill is <= max_len here, so the total needs no clamp
     chunk, nchunks = _decode_plan_span(ctx, cache.batch_size, cache.n_heads, cache.n_kv_heads,
                                        max_len, total, cache.head_dim, cache.dtype)

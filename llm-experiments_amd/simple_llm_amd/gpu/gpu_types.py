@@ -83,8 +83,6 @@ class GPUContext:
     reduction_workspace: Optional[GPUBuffer1D] = None
     # split-K workspaces of decode and prefill attention, grown on demand
     decode_workspace: Optional[torch.Tensor] = None
-    # one-launch decode steps: a zero-filled workspace per stream handle
-    step_workspaces: dict = field(default_factory=dict)
     prefill_workspace: Optional[torch.Tensor] = None
 
 
@@ -99,15 +97,20 @@ class KVCacheLayer:
     advanced on the device by every append. host_lens mirrors it exactly on
     the host (every change the kernels make is deterministic), so validation
     never has to read the device.
+
+    step_ws: workspace of the layer's one-launch decode steps (zero between
+    calls), or None where the cache's sizes do not take them.
     """
 
     def __init__(self, k_cache: GPUBuffer2D, v_cache: GPUBuffer2D,
                  lens: Optional[torch.Tensor] = None,
-                 host_lens: Optional[np.ndarray] = None):
+                 host_lens: Optional[np.ndarray] = None,
+                 step_ws: Optional[torch.Tensor] = None):
         self.k_cache = k_cache
         self.v_cache = v_cache
         self.lens = lens
         self.host_lens = host_lens
+        self.step_ws = step_ws
 
     def __repr__(self) -> str:
         return f"KVCacheLayer(k_cache={self.k_cache.shape}, v_cache={self.v_cache.shape})"

@@ -780,6 +780,99 @@ def test_one_launch_step_with_scores_that_are_not_finite(gpu_ctx, D, fill):
                 assert rel_err(got[b, h].numpy(), want.numpy()) < FP32_TOL, (b, h)
 
 
+class _Recorder:
+    """The library, noting the decode entry points that a call reaches."""
+
+    def __init__(self, lib):
+        self._lib, self.names = lib, []
+
+    def __getattr__(self, name):
+        if name.startswith("skv_append_decode_attn"):
+            self.names.append(name)
+        return getattr(self._lib, name)
+
+
+@pytest.mark.parametrize("B,H,D,T,dt,one", [
+    (15, 17, 64, 40, torch.float32, True),     # 255 pairs
+    (16, 16, 64, 40, torch.float32, False),    # 256 pairs
+    (2, 3, 64, 2048, torch.float32, True),     # 1 MB of K and V a pair
+    (2, 3, 64, 2049, torch.float32, False),
+    (2, 3, 128, 2048, torch.bfloat16, True),
+    (2, 3, 128, 2049, torch.bfloat16, False),
+    (2, 3, 48, 40, torch.float32, False),
+])
+def test_one_launch_step_route(gpu_ctx, monkeypatch, B, H, D, T, dt, one):
+    """Which calls take one launch: a rule of the cache's sizes and max_len alone."""
+    gpu = _gpu()
+    from simple_llm_amd import _lib
+    cache = gpu.kv_cache_create(gpu_ctx, gpu.KVCacheConfig(B, T, 1, H, D, dtype=dt))
+    x = [torch.randn(B, H, D, device="cuda") for _ in range(3)]
+    out = torch.empty(B, H, D, device="cuda")
+    rec = _Recorder(_lib.lib())
+    monkeypatch.setattr(_lib, "lib", lambda: rec)
+    gpu.kv_cache_append_attend(gpu_ctx, cache, 0, *x, out, max_len=T)
+    assert rec.names == ["skv_append_decode_attn_step" if one else "skv_append_decode_attn"]
+
+
+@pytest.mark.parametrize("D,dt", [(64, torch.float32), (128, torch.bfloat16)])
+def test_append_attend_has_the_same_bits_on_every_stream_and_captured(gpu_ctx, D, dt):
+    """One layer's steps on twenty streams in turn, and another's as replays of a
+    graph captured without a warm-up, with the first layer's steps between the
+    replays: outputs, fills and cache rows equal the eager ones'."""
+    gpu = _gpu()
+    B, H, T, n = 3, 4, 300, 20
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    k, v = (torch.randn(B * T, H * D, device="cuda", generator=gen).to(dt) for _ in range(2))
+    x = torch.randn(n, 3, B, H, D, device="cuda", generator=gen)
+    fills = np.array([250, 17, 0], np.int64)
+
+    def make():
+        cache = gpu.kv_cache_create(gpu_ctx, gpu.KVCacheConfig(B, T, 1, H, D, dtype=dt))
+        layer = cache.layers[0]
+        layer.k_cache.buffer.copy_(k)
+        layer.v_cache.buffer.copy_(v)
+        layer.lens.copy_(torch.from_numpy(fills))
+        layer.host_lens = fills.copy()
+        return cache, layer
+
+    def step(cache, i, out):
+        gpu.kv_cache_append_attend(gpu_ctx, cache, 0, x[i, 0], x[i, 1], x[i, 2], out, max_len=T)
+
+    eager, el = make()
+    out = torch.empty(n, B, H, D, device="cuda")
+    for i in range(n):
+        step(eager, i, out[i])
+
+    streams = [torch.cuda.Stream() for _ in range(n)]  # each waits for the one before
+    cs, sl = make()
+    got = torch.empty_like(out)
+    torch.cuda.synchronize()
+    for i, s in enumerate(streams):
+        with torch.cuda.stream(s):
+            step(cs, i, got[i])
+        s.synchronize()
+    assert torch.equal(got, out)
+    assert torch.equal(sl.k_cache.buffer, el.k_cache.buffer) and torch.equal(sl.lens, el.lens)
+
+    cg, gl = make()
+    other, ol = make()
+    inp, rep = x[0].clone(), torch.empty(B, H, D, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gpu.kv_cache_append_attend(gpu_ctx, cg, 0, inp[0], inp[1], inp[2], rep, max_len=T)
+    for i in range(n):
+        inp.copy_(x[i])
+        graph.replay()
+        step(other, i, got[i])
+        torch.cuda.synchronize()
+        assert torch.equal(rep, out[i]) and torch.equal(got[i], out[i]), i
+    for layer in (gl, ol):
+        assert torch.equal(layer.lens, el.lens)
+        assert torch.equal(layer.k_cache.buffer, el.k_cache.buffer)
+        assert torch.equal(layer.v_cache.buffer, el.v_cache.buffer)
+
+
 def test_direct_attention_split_shapes_share_a_workspace(gpu_ctx):
     """Split calls of different shapes (B x H, head dim, dtype) through one
     zero-filled workspace, interleaved: the arrival counters sit in a fixed
