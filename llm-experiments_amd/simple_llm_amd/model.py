@@ -162,10 +162,19 @@ class _PrefillBuffers:
         # (three planes), and the attention output's valid rows -> packed
         self.gather_pad = torch.zeros(3 * M, dtype=torch.int32, device=dev)
         self.gather_pk = torch.zeros(M, dtype=torch.int32, device=dev)
-        L = _lib.lib()
-        lin = max(L.skv_linear_workspace_bytes(M, n, k)
-                  for n, k in ((3 * d, d), (d, d), (mlp, d), (d, mlp)))
-        self.lin_ws = torch.zeros(max(lin, 4), dtype=torch.uint8, device=dev)
+        self.lin_ws = torch.zeros(max(_prefill_linear_bytes(M, d, mlp), 4), dtype=torch.uint8,
+                                  device=dev)
+
+
+def _prefill_linear_bytes(M: int, d: int, mlp: int) -> int:
+    """Workspace of the projections of a prefill of M rows, or of the fewer rows
+    that a packed one runs: the split products of up to 64 rows, and above 64
+    the normalised rows of the two LayerNorm projections (both read d values)."""
+    L = _lib.lib()
+    rows = [m for m in (16, 32, 48, 64) if m < M] + [min(M, 64)]
+    need = max(L.skv_linear_workspace_bytes(m, n, k) for m in rows
+               for n, k in ((3 * d, d), (d, d), (mlp, d), (d, mlp)))
+    return max(need, L.skv_linear_workspace_bytes(M, 3 * d, d)) if M > 64 else need
 
 
 class TransformerModel:
@@ -577,11 +586,13 @@ class TransformerModel:
             layer.host_lens = np.minimum(start + n_host, T)
         if all_logits:
             out = torch.empty((B, C, tm.vocab_size), device=self.ctx.device)
-            lws = torch.zeros(max(L.skv_linear_workspace_bytes(M, tm.vocab_size, d), 4),
-                              dtype=torch.uint8, device=self.ctx.device)
+            # (more than 64 rows without LayerNorm use no workspace)
+            lws = None if M > 64 else torch.zeros(
+                max(L.skv_linear_workspace_bytes(M, tm.vocab_size, d), 4), dtype=torch.uint8,
+                device=self.ctx.device)
             chk(L.skv_linear(out.data_ptr(), x, self.emb.data_ptr(), None, None, None, None, 0.0,
-                             M, tm.vocab_size, d, 0, 0, lws.data_ptr(), lws.numel(), s),
-                "skv_linear")
+                             M, tm.vocab_size, d, 0, 0, None if lws is None else lws.data_ptr(),
+                             0 if lws is None else lws.numel(), s), "skv_linear")
             return out
         # the logits of each sequence's last new row (generate.py:52 takes logits[0, -1])
         bf = self.buffers(B)

@@ -87,3 +87,20 @@ def test_backend_weight_cache_fingerprint_is_by_identity():
     assert not backend._same(fp, backend._leaves(params))
     assert backend._leaves({"embedding": params["embedding"]}) is None
     assert not backend._same(None, None)
+
+
+@pytest.mark.parametrize("B,C,d", [(8, 1024, 768), (1, 65, 128), (4, 100, 384), (2, 32, 256),
+                                   (1, 7, 64)])
+def test_prefill_workspace_is_sized_by_the_calls_that_use_it(B, C, d):
+    """The projections' workspace of a prefill: M rows of d values where
+    LayerNorm runs over more than 64 rows, and in every case room for the split
+    products of up to 64 rows (a packed prefill may run so few)."""
+    from simple_llm_amd import _lib
+    from simple_llm_amd.model import _PrefillBuffers
+
+    ws = _lib.lib().skv_linear_workspace_bytes
+    M, mlp = B * C, 4 * d
+    shapes = ((3 * d, d), (d, d), (mlp, d), (d, mlp))
+    few = max(ws(m, n, k) for m in range(1, min(M, 64) + 1) for n, k in shapes)
+    got = _PrefillBuffers("cpu", B, C, d, mlp).lin_ws.numel()
+    assert got == max(few, ws(M, 3 * d, d) if M > 64 else 0, 4)

@@ -1081,3 +1081,22 @@ def test_cache_after_run_continues(gpu_ctx, retire, direct):
     for b in live:
         want = mo.forward(params, seq[b:b + 1, :want_fill[b] + 1], 2, last=1)[0]
         assert rel_rows(lg[b:b + 1], want) < FP32_TOL, b
+
+
+def test_all_logits_prefill_allocates_its_logits_alone(gpu_ctx):
+    """The logits of more than 64 rows take no projection workspace (M * d floats
+    of LayerNorm rows, which they do not have)."""
+    from simple_llm_amd.model import TransformerModel, TransformerModelParams
+    B, C, V, d = 4, 512, 300, 512
+    m = TransformerModel(gpu_ctx, TransformerModelParams(V, d, C, 8, 1))
+    toks = np.random.default_rng(0).integers(0, V, (B, C))
+    peak = []
+    for _ in range(2):
+        cache = m.new_cache(B)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        out = m.prefill(cache, toks, all_logits=True)
+        peak.append(torch.cuda.max_memory_allocated() - base)
+        del out, cache
+    assert peak[1] <= B * C * V * 4 + (1 << 20) < B * C * (V + d) * 4
