@@ -499,7 +499,10 @@ class TransformerModel:
         d, H, D, T = tm.embedding_dim, tm.n_heads, self.head_dim, cache.max_seq_len
         M = B * C
         pos = start[:, None] + np.arange(C)[None, :]
-        pb.n_new.copy_(torch.from_numpy(n_host.astype(np.int32)))
+        # (counts that are all C are a chunk without counts)
+        ragged = int(n_host.min()) < C
+        if ragged:
+            pb.n_new.copy_(torch.from_numpy(n_host.astype(np.int32)))
         # Ragged prompts: the projections run over the valid rows only, packed
         # (row off_b + i is token i of sequence b); q, k, v are gathered into
         # the [B, C] layout of the chunk append and the attention, and the
@@ -540,7 +543,7 @@ class TransformerModel:
         x, qkv, attn, ff = pb.x.data_ptr(), pb.qkv.data_ptr(), pb.attn.data_ptr(), pb.ff.data_ptr()
         q_ptr, k_ptr, v_ptr = qkv, qkv + M * d * 4, qkv + 2 * M * d * 4
         ws, wn = pb.lin_ws.data_ptr(), pb.lin_ws.numel()
-        n_ptr = pb.n_new.data_ptr()
+        n_ptr = pb.n_new.data_ptr() if ragged else None
         ns = ctypes.c_int()
         chk(L.skv_prefill_plan(B, C, H, H, max(int((start + n_host).max()), 1), ctypes.byref(ns)),
             "skv_prefill_plan")

@@ -1100,3 +1100,38 @@ def test_all_logits_prefill_allocates_its_logits_alone(gpu_ctx):
         peak.append(torch.cuda.max_memory_allocated() - base)
         del out, cache
     assert peak[1] <= B * C * V * 4 + (1 << 20) < B * C * (V + d) * 4
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_equal_prompts_prefill_without_counts(gpu_ctx, monkeypatch, dt):
+    """Prompts that all fill the chunk are given to the attention without counts
+    (over a bf16 cache counts mean ragged chunks and smaller workgroups), with
+    the logits of the call that names them; ragged ones with."""
+    from simple_llm_amd import _lib
+    from simple_llm_amd.model import TransformerModel, TransformerModelParams
+    B, C, V, d = 3, 40, 100, 256
+    m = TransformerModel(gpu_ctx, TransformerModelParams(V, d, 64, 4, 2), kv_dtype=dt)
+    toks = np.random.default_rng(0).integers(0, V, (B, C))
+    L, counts = _lib.lib(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            f = getattr(L, name)
+            if name != "skv_append_prefill_attn":
+                return f
+            return lambda *a: (counts.append(a[7] is not None), f(*a))[1]
+
+    monkeypatch.setattr(_lib, "lib", lambda: Recorder())
+    outs = []
+    for n_new, ragged in ((None, False), (np.full(B, C), False), (np.array([C, 7, C]), True)):
+        counts.clear()
+        cache = m.new_cache(B)
+        outs.append(m.prefill(cache, toks, n_new).clone())
+        assert counts == [ragged] * 2
+        n = np.full(B, C) if n_new is None else n_new
+        for layer in cache.layers:
+            np.testing.assert_array_equal(layer.lens.cpu().numpy(), n)
+            np.testing.assert_array_equal(layer.host_lens, n)
+    assert torch.equal(outs[0], outs[1])
+    tol = FP32_TOL if dt == torch.float32 else 2e-2
+    assert rel_rows(outs[2][[0, 2]].cpu(), outs[0][[0, 2]].cpu()) < tol
