@@ -338,7 +338,7 @@ __global__ __launch_bounds__(NT) void k_sample(SampArgs a) {
     int n;
     const int off = block_excl_scan<int>(cnt, shi, &n);
     static_assert(2 * kListMax * sizeof(float) <= sizeof(phase_lds) && kListMax <= NT, "list");
-    if (n <= kListMax) {
+    if (n > 0 && n <= kListMax) {  // (min_p above 1 keeps none: dense, 0 / 0)
       listed = true;
       float* lval = reinterpret_cast<float*>(phase_lds);
       int* lidx = reinterpret_cast<int*>(phase_lds) + kListMax;

@@ -275,3 +275,15 @@ def test_short_list_edges(gpu_ctx, V, spread, step, p):
             keep = want > 0
             np.testing.assert_allclose(probs[m][keep], want[keep], rtol=1e-4, atol=1e-9)
         assert probs[m][tok[m]] > 0
+
+
+@pytest.mark.parametrize("V", [4096, 16385, 50304, 65536])
+@pytest.mark.parametrize("p", [dict(min_p=1.5), dict(min_p=1.5, top_k=40, top_p=0.9)])
+def test_min_p_above_one_keeps_nothing(gpu_ctx, V, p):
+    """No probability reaches min_p times the largest: the row's sum is 0, its
+    probabilities 0 / 0 (jax_backend.py:480-486) and its token 0, at every width."""
+    banner(f"sample min_p above 1 V={V} {p}")
+    r = np.random.default_rng(V)
+    logits = (r.standard_normal((2, V)) * 2).astype(np.float32)
+    tok, probs = run_sample(logits, np.zeros((2, 1), np.int32), np.zeros(2, np.int32), **p)
+    assert np.isnan(probs).all() and (tok == 0).all()
