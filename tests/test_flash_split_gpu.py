@@ -11,6 +11,7 @@ from conftest import banner
 from oracle import kv_oracle as ko
 from test_flash_bwd_gpu import flash_bwd
 from test_flash_fwd_gpu import flash_fwd
+from test_flash_split_oracle import BAR, flash_reference
 
 pytestmark = pytest.mark.gpu
 
@@ -51,6 +52,57 @@ def test_edges_match_oracle(gpu_ctx, N, D):
                         D, fast=fast)
         for g, w in zip(got, want):
             assert _rel(g.cpu().numpy(), w) < TOL
+
+
+# every padded head dim, in one of its load modes
+@pytest.mark.parametrize("D", [15, 16, 32, 34, 48, 52, 64, 80, 84, 96, 112, 128])
+def test_accuracy_against_float64(gpu_ctx, D):
+    """Forward and both forms of the backward within the bar that tells all six
+    partial products from any five (test_flash_split_oracle.py)."""
+    banner(f"flash split accuracy D={D}")
+    N, H = 161, 2
+    rng = np.random.default_rng(D)
+    t = [rng.standard_normal((N, H, D)).astype(np.float32) for _ in range(4)]
+    q, k, v, go = (_dev(x.reshape(N, H * D)) for x in t)
+    o, L, M = flash_fwd(q, k, v, 1, N, H, D)
+    want = [np.stack(x, 1) for x in zip(*(flash_reference(*(x[:, h] for x in t))
+                                          for h in range(H)))]
+    for fast in (False, True):
+        got = (o, *flash_bwd(q, k, v, o, L, M, go, 1, N, H, D, fast=fast))
+        for g, w, name in zip(got, want, ("o", "dq", "dk", "dv")):
+            err = _rel(g.cpu().numpy().reshape(N, H, D).astype(np.float64), w)
+            print(f"{name} rel_err={err:.2e}")
+            assert err < BAR, (name, fast)
+
+
+@pytest.mark.parametrize("D", [24, 64, 96, 128])
+def test_prefill_accuracy_against_float64(gpu_ctx, D):
+    """An fp32 cache's chunk, grouped queries after a prefix, within the same bar."""
+    from simple_llm_amd.gpu import gpu
+    banner(f"fp32 prefill accuracy D={D}")
+    B, Hq, Hkv, C, start = 2, 4, 2, 70, np.array([0, 90], np.int64)
+    T = int(start.max()) + C
+    rng = np.random.default_rng(D)
+    k, v = (rng.standard_normal((B, T, Hkv, D)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((B, C, Hq, D)).astype(np.float32)
+    cache = gpu.kv_cache_create(gpu_ctx, gpu.KVCacheConfig(B, T, 1, Hq, D, n_kv_heads=Hkv))
+    layer = cache.layers[0]
+    layer.k_cache.buffer.copy_(_dev(k.reshape(B * T, Hkv * D)))
+    layer.v_cache.buffer.copy_(_dev(v.reshape(B * T, Hkv * D)))
+    layer.lens.copy_(torch.from_numpy(start))
+    layer.host_lens = start.copy()
+    new = [_dev(np.stack([x[b, start[b]:start[b] + C] for b in range(B)])) for x in (k, v)]
+    out = torch.empty(B, C, Hq, D, device="cuda")
+    gpu.kv_cache_prefill(gpu_ctx, cache, 0, *new, _dev(q), out)
+    got = out.cpu().numpy().astype(np.float64)
+    for b in range(B):
+        n = int(start[b]) + C
+        for h in range(Hq):
+            s = (q[b, :, h].astype(np.float64) @ k[b, :n, h // 2].astype(np.float64).T) / D ** 0.5
+            s[np.arange(n)[None] > start[b] + np.arange(C)[:, None]] = -np.inf
+            e = np.exp(s - s.max(1, keepdims=True))
+            want = (e / e.sum(1, keepdims=True)) @ v[b, :n, h // 2].astype(np.float64)
+            assert _rel(got[b, :, h], want) < BAR, (b, h)
 
 
 def _reference(q, k, v, go):

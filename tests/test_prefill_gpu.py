@@ -322,7 +322,11 @@ def test_workgroup_sizes_give_the_same_bits(D, G, C):
     L = _lib.lib()
     s = torch.cuda.current_stream().cuda_stream
     rows = (C * G + 255) // 256  # 256-row tiles of a (sequence, kv head)
-    B, Hkv = 4, -(-256 // (4 * rows))  # a full round: at least seven eighths of the CUs
+    # Four sequences' workgroups on one to four full rounds of the CUs, at both
+    # split counts: the call without counts keeps 256 rows.
+    B = 4
+    Hkv = next(n for n in range(1, 257)
+               if all(8 * w >= 7 * 256 * -(-w // 256) for w in (4 * rows * n, 12 * rows * n)))
     Hq, T = Hkv * G, 500 + C
     gen = torch.Generator(device="cuda").manual_seed(D * 1000 + C)
     k = torch.randn(B, T, Hkv, D, device="cuda", generator=gen).to(torch.bfloat16)
