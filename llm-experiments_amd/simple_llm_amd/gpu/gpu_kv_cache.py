@@ -430,9 +430,12 @@ def kv_cache_append_attend(ctx: GPUContext, cache: KVCache, layer_idx: int, new_
     Appends new_k/new_v ([batch_size, n_kv_heads, head_dim], or flat) at each
     sequence's fill (full sequences are skipped), then attends q
     ([batch_size, n_heads, head_dim]) over the fills including the new token,
-    writing out. The same results as the two calls, without the separate
-    append launch (skv_append_decode_attn). max_len bounds the fills after
-    the append (default: the host mirror's). Returns the new fills.
+    writing out. The same cache and fills as the two calls, without the
+    separate append launch. out has their bits too (skv_append_decode_attn),
+    except where few short rows take one launch (skv_append_decode_attn_step,
+    see _STEP_PAIRS), which sums a row in another order: within fp32 rounding
+    there. max_len bounds the fills after the append (default: the host
+    mirror's). Returns the new fills.
     """
     _check_layer(cache, layer_idx)
     layer = cache.layers[layer_idx]
@@ -550,7 +553,7 @@ def kv_cache_prefill(ctx: GPUContext, cache: KVCache, layer_idx: int, new_k: tor
     prefix). The layer's fills advance by n_new. Returns the new fills.
 
     A bfloat16 cache runs the bf16 MFMA prefill; a float32 cache runs every
-    product in fp32 (float32 q and out).
+    product with fp32 accuracy (float32 q and out).
 
     Raises ValueError (before any GPU work) on a bad layer, shapes, a chunk
     that would overflow a sequence ("Cache is full"), a paged cache, or a
