@@ -7,7 +7,7 @@
 // flash_attention_backward (gpu/gpu_pass_backward.py:445-580).
 //
 // What bounds these kernels: the matrix cores do a third of the fp32 MFMA
-// kernels' cycles, and the vector instructions that split the operands (5.5 a
+// kernels' cycles, and the vector instructions that split the operands (6.5 a
 // value) and form the probabilities come to about as many; the forward at B=8,
 // N=2048, H=16, D=64 is 56 % MFMA busy, at the 1.83 GHz that the card's power
 // allows this mix (the fp32 form: 77 % at 2.4 GHz).
@@ -176,11 +176,11 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
 // one after it loaded into registers, and the second half of P is split while
 // the first is multiplied, so most vector instructions run between MFMAs.
 // Measured on MI355X against the fp32 MFMA form (B, N, H, D; us): 8, 2048, 16,
-// 64: 570 -> 388; 2, 1024, 12, 64: 78 -> 49; 2, 2048, 16, 128: 330 -> 220; 5,
-// 1605, 8, 96: 254 -> 134; 4, 333, 8, 48: 30.5 -> 19.6. Relative 2-norm error
+// 64: 570 -> 403; 2, 1024, 12, 64: 78 -> 51; 2, 2048, 16, 128: 330 -> 222; 5,
+// 1605, 8, 96: 254 -> 139; 4, 333, 8, 48: 30.5 -> 19.9. Relative 2-norm error
 // against float64 at N = 150, D = 64: 2.2e-7 -> 1.5e-7. With 64 keys a step in
-// one LDS stage: 399 for the first; with 8 wavefronts a workgroup 374, but 66
-// for the second and 145 for the fourth.
+// one LDS stage: 399 for the first, against 388 at the time; with 8 wavefronts
+// a workgroup 374, but 66 for the second and 145 for the fourth.
 // ---------------------------------------------------------------------------
 template <int D, int MODE>
 __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(FfwdArgs a) {
@@ -440,11 +440,11 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 // that the dK/dV kernel wrote (the same bits: the partial products are taken
 // in the same order).
 // Measured on MI355X against the fp32 MFMA forms (B, N, H, D; us): 8, 2048, 16,
-// 64: 1520 -> 1110; 2, 1024, 12, 64: 203 -> 138; 2, 2048, 16, 128: 1055 -> 700;
-// 5, 1605, 8, 96: 707 -> 465; 4, 333, 8, 48: 81 -> 51. The largest relative
+// 64: 1520 -> 1125; 2, 1024, 12, 64: 203 -> 140; 2, 2048, 16, 128: 1055 -> 709;
+// 5, 1605, 8, 96: 707 -> 483; 4, 333, 8, 48: 81 -> 51. The largest relative
 // 2-norm error against float64 of dQ, dK and dV at the first: 1.1e-6 -> 8.3e-7.
 // Before P and dS were formed under the products, and with dQ's K 32 rows a
-// step: 1160, 164 and 60 for the first, second and last.
+// step: 1160, 164 and 60 for the first, second and last, against 1110, 138 and 51.
 // ---------------------------------------------------------------------------
 
 // The operands are split as 2^16 x here, so that what the chain of products

@@ -11,8 +11,8 @@
 // takes six partial products on v_mfma_f32_32x32x16_bf16 (split_bf16.h).
 // Measured on MI355X against the fp32 MFMA form of the same kernel (128 x 128
 // tiles, one LDS stage): 2048 x 50304 x 768 1390 -> 853 us (186 TFLOP/s),
-// 2048 x 3072 x 768 with LayerNorm 137 -> 67 us, 2048 x 768 x 3072 220 -> 79
-// us, 111 x 640 x 2560 192 -> 48 us; error against float64 (relative
+// 2048 x 3072 x 768 with LayerNorm 137 -> 69 us, 2048 x 768 x 3072 220 -> 84
+// us, 111 x 640 x 2560 192 -> 49 us; error against float64 (relative
 // 2-norm) 5.0e-7 -> 4.2e-7 at K = 768 and 9.9e-7 -> 8.6e-7 at K = 3072.
 // Outputs that are not finite (an infinity, or a value too large to split,
 // among the operands) are computed again on v_mfma_f32_32x32x2_f32, which
@@ -423,7 +423,8 @@ int gemm_linear(float* y, const float* x, const float* w_t, const float* bias,
     a.ln_g = a.ln_b = nullptr;
   }
   if (lng) return launch_gemm<64, 64, 32, 32, false, true>(a, s);
-  // Tiles by how they fill the chip's 256 CUs (measured on MI355X, us):
+  // Tiles by how they fill the chip's 256 CUs (measured on MI355X, us, all of
+  // them before the operands were scaled, which costs up to 6 %):
   //  - 256 x 128 where there are more than two rounds of them: the fewest
   //    values split per product (2048 x 50304 x 768: 853, 128 x 64 955, 64 x
   //    64 1128). With fewer, its long workgroups leave CUs idle (2048 x 2304 x
