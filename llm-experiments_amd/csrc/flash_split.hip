@@ -182,6 +182,7 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
 // one LDS stage: 399 for the first, against 388 at the time; with 8 wavefronts
 // a workgroup 374, but 66 for the second and 145 for the fourth.
 // ---------------------------------------------------------------------------
+constexpr float kQueryScale = 0x1p40f, kScoreUnscale = 0x1p-64f;
 template <int D, int MODE>
 __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(FfwdArgs a) {
   constexpr int KB = D / 16;             // k-blocks of Q K^T
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
   float m_run = -INFINITY, m_true = -INFINITY, l = 0.f;
 
   // The online softmax of the piece at key0: s holds its scores in log2 units
-  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query) times 2^48, and
+  // (key key0 + 8 (r / 4) + 4 hf + r % 4 of this lane's query) times 2^64, and
   // gets the probabilities times 2^24.
   auto softmax = [&](f32x16& s, int key0) {
     // A piece wholly at or below the diagonal of a wave whose 32 queries are
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-    tmax = xor32_max(tmax) * kSplitUnscale;  // both halves hold the same query
+    tmax = xor32_max(tmax) * kScoreUnscale;  // both halves hold the same query
     m_true = fmaxf(m_true, tmax);
     const bool upd = tmax > m_run + 8.f;  // also true on the first piece with a key
     if (__ballot(upd) != 0ull) {          // wave-uniform branch
@@ -254,14 +255,16 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
     const float m_use = m_run == -INFINITY ? 0.f : m_run;  // nothing unmasked yet
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(fmaf(s[r], kSplitUnscale, -m_use));
+      s[r] = fast_exp2(fmaf(s[r], kScoreUnscale, -m_use));
       l += s[r];
       s[r] *= kSplitScale;
     }
   };
 
-  bf16x8 qf[KB][3];  // the query, so that the scores come out in log2 units
-  const float qs = a.sl2 * kSplitScale;
+  // the query, so that the scores come out in log2 units: rounded, so its
+  // smallest values have more bits to keep than an operand's own
+  bf16x8 qf[KB][3];
+  const float qs = a.sl2 * kQueryScale;
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb)
     split8(load4m<MODE>(qp, 16 * kb + 8 * hf, RS) * qs,
@@ -447,12 +450,13 @@ __global__ __launch_bounds__(kThreads, D <= 96 ? 2 : 1) void k_flash_fwd_split(F
 // step: 1160, 164 and 60 for the first, second and last, against 1110, 138 and 51.
 // ---------------------------------------------------------------------------
 
-// The operands are split as 2^16 x here, so that what the chain of products
-// carries, 2^32 for S and dP, 2^48 for dS (of dP and 2^16 P) and 2^64 for dK
-// and dQ, leaves room for large gradients (a sum past the largest float takes
-// the fp32 form); operands below 2^-142 (fp32 subnormals) keep fewer bits.
-constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
-constexpr float kProdScale = 0x1p32f, kDsUnscale = 0x1p-48f, kGradUnscale = 0x1p-64f;
+// What the chain of products carries: 2^48 for S and dP, 2^16 for P (its
+// smallest normal value keeps every bit), so 2^40 for dV, 2^64 for dS and 2^88
+// for dK and dQ formed from it. Sums past the largest float, gradients from
+// 2^40, take the fp32 form.
+constexpr float kProdScale = kSplitScale * kSplitScale;
+constexpr float kPScale = 0x1p16f, kDvUnscale = 0x1p-40f;
+constexpr float kDsUnscale = 0x1p-64f, kGradUnscale = 0x1p-88f;
 
 // c += A B as mfma_split(b, a, c) orders the partial products of its factors.
 __device__ __forceinline__ f32x16 mfma_split_swapped(const bf16x8 (&a)[3], const bf16x8 (&b)[3],
@@ -513,11 +517,11 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int d0 = 16 * kb + 8 * hf;
-    split8(load4m<MODE>(a.k + koff, d0, RS) * kScale,
-           load4m<MODE>(a.k + koff, d0 + 4, RS) * kScale, kf[kb]);
+    split8(load4m<MODE>(a.k + koff, d0, RS) * kSplitScale,
+           load4m<MODE>(a.k + koff, d0 + 4, RS) * kSplitScale, kf[kb]);
     bf16x8 vf[3];
-    split8(load4m<MODE>(a.v + koff, d0, RS) * kScale,
-           load4m<MODE>(a.v + koff, d0 + 4, RS) * kScale, vf);
+    split8(load4m<MODE>(a.v + koff, d0, RS) * kSplitScale,
+           load4m<MODE>(a.v + koff, d0 + 4, RS) * kSplitScale, vf);
 #pragma unroll
     for (int p = 0; p < 3; ++p) sm.v[wave][kb][p][lane] = vf[p];
   }
@@ -551,15 +555,14 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
     if (threadIdx.x < 32) {  // statistics of query j * 32 + threadIdx.x, clamped
       const size_t sr = (size_t)(b * N + min(j * 32 + (int)threadIdx.x, N - 1)) * H + h;
       m2 = a.M[sr] * LOG2E;
-      il = 1.f / a.L[sr] * kScale;
+      il = 1.f / a.L[sr] * kPScale;
       dl = a.delta[sr] * kProdScale;
     }
   };
-  const float sl2 = a.sl2 * kUnscale;
+  const float sl2 = a.sl2 * kSplitUnscale;
   // One piece. s[r], dp[r]: query q0 + 8(r/4) + 4hf + r%4, key krow. The
   // vector work stands between products that do not wait for it: P is formed
-  // and split under dP = dO V^T, dS under dV += P^T dO. S and dP carry 2^32,
-  // P (by il) 2^16 and dS, of P and dP, 2^48.
+  // and split under dP = dO V^T, dS under dV += P^T dO.
   auto piece = [&](auto interior, int q0) {
     f32x16 s = f32x16{}, dp = f32x16{};
     bf16x8 pf[2][3], df[2][3];
@@ -633,7 +636,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
   for (int j = j0; j < pieces; ++j) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sm.q : sm.d, kScale);
+    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sm.q : sm.d, kSplitScale);
     if (threadIdx.x < 32) {
       sm.m2[threadIdx.x] = m2;
       sm.il[threadIdx.x] = il;
@@ -661,7 +664,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dkv_split(Fb
       if (key < N && d < RS) {
         const size_t off = row_off(b, key, N, H, h, RS) + d;
         a.dk[off] = dka[dt][r] * kGradUnscale * a.scale;
-        a.dv[off] = dva[dt][r] * kUnscale;
+        a.dv[off] = dva[dt][r] * kDvUnscale;
         bad |= !(finite(dva[dt][r]) && finite(dka[dt][r]));
       }
     }
@@ -837,10 +840,10 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int d0 = 16 * kb + 8 * hf;
-    split8(load4m<MODE>(a.q + qoff, d0, RS) * kScale,
-           load4m<MODE>(a.q + qoff, d0 + 4, RS) * kScale, qf[kb]);
-    split8(load4m<MODE>(a.dout + qoff, d0, RS) * kScale,
-           load4m<MODE>(a.dout + qoff, d0 + 4, RS) * kScale, df[kb]);
+    split8(load4m<MODE>(a.q + qoff, d0, RS) * kSplitScale,
+           load4m<MODE>(a.q + qoff, d0 + 4, RS) * kSplitScale, qf[kb]);
+    split8(load4m<MODE>(a.dout + qoff, d0, RS) * kSplitScale,
+           load4m<MODE>(a.dout + qoff, d0 + 4, RS) * kSplitScale, df[kb]);
   }
   f32x16 acc[DT];
 #pragma unroll
@@ -848,7 +851,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
   const int pieces = (min(blk * kRows + kRows, N) + 31) / 32;
   const int wq_last = wq0 < N ? min(wq0 + 31, N - 1) : -1;  // -1: the wave has no query
 
-  // dS of a piece from S and dP, which carry 2^32 (prod) and give 2^48, or 1
+  // dS of a piece from S and dP, which carry prod (1 / unit), P taking p_scale
   auto to_ds = [&](const f32x16& s, f32x16& dp, int key0, float unit, float prod, float p_scale) {
     const float sl2 = a.sl2 * unit, dlp = dl * prod, ilp = il * p_scale;
 #pragma unroll
@@ -869,7 +872,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
   for (int j = 0; j < pieces; ++j) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sK : sV, kScale);
+    for (int i = 0; i < 2 * NV; ++i) st[i / NV].store(i % NV, i < NV ? sK : sV, kSplitScale);
     __syncthreads();
     if (j + 1 < pieces) load_piece(j + 1);
     const int key0 = j * 32;
@@ -883,7 +886,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void k_fbwd_dq_split(Fbw
       s = mfma_split_swapped(ka, qf[kb], s);
       dp = mfma_split_swapped(va, df[kb], dp);
     }
-    to_ds(s, dp, key0, kUnscale, kProdScale, kScale);
+    to_ds(s, dp, key0, kSplitUnscale, kProdScale, kPScale);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       bf16x8 f[3];
@@ -976,7 +979,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
     constexpr int F = decltype(fc)::value;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NV; ++i) st.store(i, sK, kScale);
+    for (int i = 0; i < NV; ++i) st.store(i, sK, kSplitScale);
     __syncthreads();
     if (j + 1 < steps) {
 #pragma unroll
@@ -992,7 +995,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         bf16x8 f[3];
-        split8(cur[2 * kk] * kScale, cur[2 * kk + 1] * kScale, f);
+        split8(cur[2 * kk] * kSplitScale, cur[2 * kk + 1] * kSplitScale, f);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           bf16x8 kt[3];
@@ -1006,7 +1009,7 @@ __global__ __launch_bounds__(kThreads) void k_fbwd_dq_ds_split(FbwdArgs a) {
     step(std::integral_constant<int, 0>{}, j);
     if (j + 1 < steps) step(std::integral_constant<int, 1>{}, j + 1);
   }
-  finish_dq<DT, MODE>(a, acc, kUnscale, row_off(b, qrow, N, H, h, RS), qok, wq_last, kh, rs, RS, c,
+  finish_dq<DT, MODE>(a, acc, kSplitUnscale, row_off(b, qrow, N, H, h, RS), qok, wq_last, kh, rs, RS, c,
                       hf, [&](int key0) {
     f32x4 x[4];
     load_ds(key0, x);
